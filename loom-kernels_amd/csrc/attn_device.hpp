@@ -11,6 +11,7 @@ namespace loom_dev {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -93,6 +94,14 @@ __device__ __forceinline__ void lds_load16_at(__amdgpu_buffer_rsrc_t r, uint32_t
                                               int byte_offset) {
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_addr);
   asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, 0 offen lds" ::"v"(byte_offset),
+               "s"(m0), "s"(r)
+               : "m0", "memory");
+}
+// 4 bytes per lane, otherwise as lds_load16 (lane i's bytes at lds + 4 i).
+__device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t r, void *lds, int byte_offset) {
+  const uint32_t m0 =
+      __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)lds);
+  asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dword %0, %2, 0 offen lds" ::"v"(byte_offset),
                "s"(m0), "s"(r)
                : "m0", "memory");
 }
@@ -225,6 +234,33 @@ __device__ __forceinline__ int wave_max_i32(int x) {
   return x;
 }
 
+// Inclusive prefix over the wave in registers (DPP row shifts within 16 lanes,
+// then row broadcasts): saturating unsigned sum, and max of non-negative ints.
+__device__ __forceinline__ uint32_t wave_incl_add_sat_u32(uint32_t x) {
+#define LOOM_SCAN_STEP(ctrl, rows)                                                       \
+  x = __builtin_elementwise_add_sat(                                                     \
+      x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, rows, 0xf, false))
+  LOOM_SCAN_STEP(0x111, 0xf);
+  LOOM_SCAN_STEP(0x112, 0xf);
+  LOOM_SCAN_STEP(0x114, 0xf);
+  LOOM_SCAN_STEP(0x118, 0xf);
+  LOOM_SCAN_STEP(0x142, 0xa);
+  LOOM_SCAN_STEP(0x143, 0xc);
+#undef LOOM_SCAN_STEP
+  return x;
+}
+__device__ __forceinline__ int32_t wave_incl_max_i32(int32_t x) {
+#define LOOM_SCAN_STEP(ctrl, rows) x = max(x, __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false))
+  LOOM_SCAN_STEP(0x111, 0xf);
+  LOOM_SCAN_STEP(0x112, 0xf);
+  LOOM_SCAN_STEP(0x114, 0xf);
+  LOOM_SCAN_STEP(0x118, 0xf);
+  LOOM_SCAN_STEP(0x142, 0xa);
+  LOOM_SCAN_STEP(0x143, 0xc);
+#undef LOOM_SCAN_STEP
+  return x;
+}
+
 __device__ __forceinline__ int64_t wave_incl_scan64(int64_t x, int lane) {
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -274,6 +310,18 @@ __device__ __forceinline__ float quad_sum(float x) {
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
                                                   false);
   x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// Max / sum over the two 32-lane halves of a wave (lanes l and l ^ 32).
+__device__ __forceinline__ float half_max(float x) {
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float half_sum(float x) {
   const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
                                                   false);
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);

@@ -93,10 +93,248 @@ struct PrefillArgs {
   const float *kv_scales;
 };
 
+// ---- locating a workgroup's tile ------------------------------------------------
+// The tile of workgroup blockIdx.x and the request that owns it (wave-uniform).
+struct TileLoc {
+  int kvh;
+  int tile0;              // tile within the request's columns
+  int32_t qs, qe;         // the request's qo_indptr pair
+  int32_t ps, pe;         // its page (ragged: kv) indptr pair
+  int32_t tl;             // its last page's rows (paged)
+  int32_t fbeg;           // first flattened column it owns
+  int32_t ipB;            // indptr[batch]
+};
+
 // Tile count given to a request whose qo range is malformed: larger than any
 // tile index, so neither it nor any later request owns a tile (the reference's
 // request search returns at the first malformed range, prefill.rs:303-313).
 constexpr int64_t kNoTiles = (int64_t)1 << 50;
+
+template <int W>
+struct LocateSmem {
+  int64_t wave_tot[W];
+  int32_t wave_max[W];
+  int32_t req;
+  int32_t tile0;
+  // the located request's qo_indptr pair, page (or kv) indptr pair, tail, and
+  // the first flattened column it owns
+  int32_t meta[6];
+};
+
+// Finds the tile of this workgroup (TC flattened columns per tile) and applies
+// the global guards (prefill.rs:293-300 paged, :102-108 ragged); false: no
+// tile, or a failed guard.
+//
+// Tiles come in reverse order: a request's later rows see longer causal
+// ranges, so the heaviest tiles are dispatched first and the launch does not
+// end with a few long tiles running alone (the grid's excess workgroups, which
+// find no tile, come first and exit at once).  Workgroup b runs on XCD b % 8;
+// with the kv-head fastest, each XCD keeps to a fixed set of kv-heads, whose
+// K/V its L2 shares across tiles.
+//
+// The metadata comes in as few dependent round trips as possible: every
+// request's qo range, page (kv) range and tail are loaded together and the
+// guards applied afterwards.  Paged (prefill.rs:303-313): rows belong to the
+// requests before the first malformed qo range.  Ragged (prefill.rs:111-137):
+// row q belongs to the first request r with q < qo_indptr[r+1], i.e. r owns
+// the rows from max(qo_indptr[r], max(qo_indptr[1..r])) to qo_indptr[r+1], and
+// a request failing its guards keeps its rows' sentinels.
+//
+// Up to 64 requests every wave holds the whole table, one request per lane,
+// and finds the tile by itself with register scans: no LDS and no barrier on
+// the way (16 requests of 256 BF16 rows, GQA4 32/8: 35.0 -> 34.3 us; 1 x 1024
+// 22.3 -> 21.5, 1 x 512 13.8 -> 12.9; a batch of two on row tiles 14.2 -> 13.5).
+template <int W, bool RAGGED, int TC, bool INTERLEAVE>
+__device__ __forceinline__ bool locate_tile(const PrefillArgs &a, LocateSmem<W> &sm, TileLoc &t) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  t.kvh = (int)(blockIdx.x % a.hkv);
+  const int64_t n_tiles = (int64_t)(gridDim.x / a.hkv), m = blockIdx.x / a.hkv;
+  int64_t rank = m;
+  if (a.tile_layer > 0) {
+    // Serpentine: every other layer of tile_layer workgroups (one per CU of
+    // the XCDs this kv-head runs on) takes its tiles in reverse, so a CU's
+    // successive workgroups pair heavy tiles with light ones instead of
+    // stacking the heaviest of every layer.
+    const int64_t L = a.tile_layer, layer = m / L, c = m - layer * L;
+    const int64_t width = min(L, n_tiles - layer * L);
+    rank = layer * L + ((layer & 1) ? width - 1 - c : c);
+  }
+  const int64_t tile = n_tiles - 1 - rank;
+  const bool interleave = INTERLEAVE && a.tile_interleave != 0;
+  auto guards = [&](int32_t qo0, int32_t qoB, int32_t ip0, int32_t ipB) {
+    t.ipB = ipB;
+    if constexpr (RAGGED) return qo0 == 0 && qoB == a.nnz && ip0 == 0 && ipB == a.nnz_kv;
+    return qo0 == 0 && qoB == a.nnz && ip0 == 0 && ipB >= 0 &&
+           (a.indices_capacity ? (int64_t)ipB <= a.n_indices : (int64_t)ipB == a.n_indices);
+  };
+  // Tiles of a request that owns the rows [lo, s1) (ragged: lo past earlier
+  // requests' rows); kNoTiles where the paged search ends.
+  auto count = [&](int32_t s0, int32_t s1, int32_t p0, int32_t p1, int32_t lo) -> int64_t {
+    if constexpr (RAGGED) {
+      const bool ok = s0 >= 0 && s1 > s0 && s1 <= a.nnz && p0 >= 0 && p1 > p0 && p1 <= a.nnz_kv &&
+                      s1 - s0 <= p1 - p0;
+      return ok && s1 > lo ? ((int64_t)(s1 - lo) * a.group + TC - 1) / TC : 0;
+    }
+    return (s0 >= 0 && s1 > s0 && s1 <= a.nnz) ? ((int64_t)(s1 - s0) * a.group + TC - 1) / TC
+                                               : kNoTiles;
+  };
+
+  if (a.batch <= 64) {
+    int32_t s0 = 0, s1 = 0, p0 = 0, p1 = 0, t1 = 0;
+    const bool in = lane < a.batch;
+    if (in) {
+      s0 = a.qo[lane];
+      s1 = a.qo[lane + 1];
+      p0 = a.indptr[lane];
+      p1 = a.indptr[lane + 1];
+      if constexpr (!RAGGED) t1 = a.last[lane];
+    }
+    int32_t lo = s0;
+    if constexpr (RAGGED) {
+      const int32_t ends = wave_incl_max_i32(in ? s1 : 0);  // running max of the qo ends
+      lo = max(s0, __builtin_amdgcn_update_dpp(0, ends, 0x138, 0xf, 0xf, false));  // (of lane - 1)
+    }
+    const int64_t cnt64 = in ? count(s0, s1, p0, p1, lo) : 0;
+    // (saturated: a count or a prefix past UINT32_MAX lies past every tile)
+    const uint32_t cnt = (uint32_t)min<int64_t>(cnt64, (int64_t)UINT32_MAX);
+    bool mine;
+    if (interleave) {
+      // Tile `rank` of all requests' tiles in order of their distance from
+      // their request's end (after the grid's excess workgroups): the j-th of
+      // the tiles k from their request's end, where k is the largest with
+      // F(k) = sum of min(k, count) <= it and j counts requests with more
+      // than k tiles in request order; requests from the first malformed qo
+      // range on own no tile.  Each lane evaluates F at one k, so a round
+      // narrows the range of k 64-fold.
+      const uint64_t badm = __builtin_amdgcn_ballot_w64(in && cnt64 == kNoTiles);
+      const int first_bad = badm ? __builtin_ctzll(badm) : 64;
+      const uint32_t c = (in && lane < first_bad) ? cnt : 0u;
+      auto F = [&](uint32_t k) {
+        uint32_t f = 0;
+        for (int r = 0; r < a.batch; ++r)
+          f = __builtin_elementwise_add_sat(
+              f, (uint32_t)min(k, (uint32_t)__builtin_amdgcn_readlane((int)c, r)));
+        return f;
+      };
+      // F at one wave-uniform k
+      auto F1 = [&](uint32_t k) {
+        return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_add_sat_u32(min(k, c)), 63);
+      };
+      const int64_t rr = rank - (n_tiles - (int64_t)F1(UINT32_MAX));
+      if (rr < 0) return false;
+      uint32_t base = 0, span = (uint32_t)n_tiles;  // k in [base, base + span)
+      while (span > 1) {
+        const uint32_t st = (span + 63) >> 6;
+        const uint64_t below = __builtin_amdgcn_ballot_w64(lane * st < span &&
+                                                           (int64_t)F(base + lane * st) <= rr);
+        const uint32_t n = (uint32_t)__builtin_popcountll(below) - 1u;  // F(base) <= rr always
+        base += n * st;
+        span = min(st, span - n * st);
+      }
+      const int j = (int)(rr - (int64_t)F1(base));
+      const uint64_t more = __builtin_amdgcn_ballot_w64(c > base);
+      const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(more >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)more, 0u));
+      mine = c > base && before == j;
+      t.tile0 = (int)(c - 1u - base);
+    } else {
+      const uint32_t incl = wave_incl_add_sat_u32(cnt);
+      const uint32_t excl = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x138, 0xf, 0xf, false);
+      mine = in && cnt64 != kNoTiles && tile < (int64_t)incl && tile >= (int64_t)excl;
+      t.tile0 = (int)(tile - (int64_t)excl);
+    }
+    const uint64_t who = __builtin_amdgcn_ballot_w64(mine);
+    const int B1 = a.batch - 1;
+    if (!guards(__builtin_amdgcn_readlane(s0, 0), __builtin_amdgcn_readlane(s1, B1),
+                __builtin_amdgcn_readlane(p0, 0), __builtin_amdgcn_readlane(p1, B1)))
+      return false;
+    if (!who) return false;
+    const int w = __builtin_ctzll(who);
+    t.tile0 = __builtin_amdgcn_readlane(t.tile0, w);
+    t.qs = __builtin_amdgcn_readlane(s0, w);
+    t.qe = __builtin_amdgcn_readlane(s1, w);
+    t.ps = __builtin_amdgcn_readlane(p0, w);
+    t.pe = __builtin_amdgcn_readlane(p1, w);
+    t.tl = __builtin_amdgcn_readlane(t1, w);
+    t.fbeg = RAGGED ? (__builtin_amdgcn_readlane(lo, w) - t.qs) * a.group : 0;
+    return true;
+  }
+
+  // Larger batches: a workgroup-wide prefix of the requests' tile counts.
+  const int32_t qo0 = a.qo[0], qoB = a.qo[a.batch];
+  const int32_t ip0 = a.indptr[0], ipB = a.indptr[a.batch];
+  if (tid == 0) sm.req = -1;
+  int64_t carry = 0;
+  int32_t carry_max = 0;
+  for (int base = 0; base < a.batch; base += W * 64) {
+    const int r = base + tid;
+    int32_t s0 = 0, s1 = 0, p0 = 0, p1 = 0, t1 = 0;
+    if (r < a.batch) {
+      s0 = a.qo[r];
+      s1 = a.qo[r + 1];
+      p0 = a.indptr[r];
+      p1 = a.indptr[r + 1];
+      if constexpr (!RAGGED) t1 = a.last[r];
+    }
+    int32_t lo = s0;
+    if constexpr (RAGGED) {
+      // exclusive running max of the qo ends before r
+      int32_t x = r < a.batch ? s1 : INT32_MIN;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x = max(x, y);
+      }
+      if (lane == 63) sm.wave_max[wave] = x;
+      __syncthreads();
+      int32_t before = carry_max, blk = carry_max;
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        before = i < wave ? max(before, sm.wave_max[i]) : before;
+        blk = max(blk, sm.wave_max[i]);
+      }
+      const int32_t up = __shfl_up(x, 1, 64);
+      lo = max(s0, lane > 0 ? max(before, up) : before);
+      carry_max = blk;
+    }
+    const int64_t cnt = r < a.batch ? count(s0, s1, p0, p1, lo) : 0;
+    const int64_t x = wave_incl_scan64(cnt, lane);
+    if (lane == 63) sm.wave_tot[wave] = x;
+    __syncthreads();
+    int64_t before = 0, tot = 0;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const int64_t y = sm.wave_tot[i];
+      before += (i < wave) ? y : 0;
+      tot += y;
+    }
+    const int64_t incl = carry + before + x;
+    if (r < a.batch && tile < incl && tile >= incl - cnt && cnt != kNoTiles) {
+      sm.req = r;
+      sm.tile0 = (int32_t)(tile - (incl - cnt));
+      sm.meta[0] = s0;
+      sm.meta[1] = s1;
+      sm.meta[2] = p0;
+      sm.meta[3] = p1;
+      sm.meta[4] = t1;
+      sm.meta[5] = RAGGED ? (lo - s0) * a.group : 0;
+    }
+    carry += tot;
+    __syncthreads();
+    if (carry > tile) break;
+  }
+  if (!guards(qo0, qoB, ip0, ipB)) return false;
+  if (uni(sm.req) < 0) return false;
+  t.tile0 = uni(sm.tile0);
+  t.qs = uni(sm.meta[0]);
+  t.qe = uni(sm.meta[1]);
+  t.ps = uni(sm.meta[2]);
+  t.pe = uni(sm.meta[3]);
+  t.tl = uni(sm.meta[4]);
+  t.fbeg = uni(sm.meta[5]);
+  return true;
+}
 
 // Pages in flight per wave (32 VGPRs each): 16-wave workgroups have 128
 // registers per lane and no room for a prefetch; 4 and 8 waves use two (deeper
@@ -108,13 +346,7 @@ constexpr int prefill_depth(int w) { return w >= 16 ? 1 : LOOM_PREFILL_DEPTH; }
 
 template <int W, bool SH, int LT = 0>
 struct PrefillSmem {
-  int64_t wave_tot[W];
-  int32_t wave_max[W];
-  int32_t req;
-  int32_t tile0;
-  // the located request's qo_indptr pair, page (or kv) indptr pair, tail, and
-  // the first flattened column it owns
-  int32_t meta[6];
+  LocateSmem<W> loc;
   // MFMA B fragments of 16 query columns (per wave: SH; long tiles keep them
   // in registers)
   u32x4 qfrag[LT ? 0 : SH ? W : 1][4][64];
@@ -613,6 +845,353 @@ struct LongWave {
   }
 };
 
+// ---- pipelined long tiles (LOOM_PAGED_PREFILL_LONG_TILE, 128 columns) -----------
+// A workgroup owns 32 * NW flattened columns, two 16-column tiles per wave,
+// and walks the whole causal range in 32-token blocks (two 16-row blocks),
+// which are loaded straight into an LDS ring (buffer loads to LDS: no VGPRs or
+// LDS stores).  G groups of NW waves own the same columns and split the blocks
+// (block b to group b % G); their states merge at the end.
+//
+// Bound and shape.  A 16x16x32 MFMA takes 16 cycles of the SIMD's matrix core
+// and holds its vector issue for 8 of them, an exponential for 8, other vector
+// instructions 4 (measured with register-only loops), and a wave issues in
+// order.  Per wave and block: 32 MFMAs (512 cycles), 16 exponentials and about
+// 35 other vector instructions, which fit beside the MFMAs only if they are
+// issued between them.  Hence: the products of one block, the softmax of the
+// next and the scores of the one after interleaved by hand (pin()); no maximum
+// per block; normalizer sums by dot products with ones; page addresses
+// computed per 64 blocks, one per lane; whole rows per load instruction.  Two
+// waves per SIMD (235 registers).  Tried with 32x32x16 MFMAs: a tenth faster
+// on cool data (zeros), but their energy per flop is higher and random data
+// holds the card at its power limit from about 4096 rows on, where they lost 3%.
+// Measured against the plain long tiles: see the plan's rule.
+//
+// acc[t][e][i] = O[column of tile t][dim 16 e + 4 quad + i].
+//
+// Normalizer past which a column's reference max is refreshed (see step()).
+constexpr float kRefreshNormalizer = 16777216.0f;
+
+// HL: P enters the product as a BF16 high part and a BF16 residual (two MFMAs
+// per block of V), so the weights carry 16 significant bits and the
+// normalizer sums them in FP32.  Otherwise P is rounded once to BF16 and the
+// normalizer sums the rounded weights.
+template <int NW, bool FP8, bool HL, int G>
+struct PipeWave {
+  const PrefillArgs &a;
+  int lane, col, quad;
+  int64_t end_col[2];  // causal end (exclusive) of the lane's column of each tile, 0 if unused
+  int64_t full_end;    // smallest causal end of the wave's valid columns
+  float nmax[2];       // negated reference max (log2 domain, scaled); +inf: none yet
+  float lsum[2];       // normalizer over the lane's quarter of the tokens
+  f32x4 acc[2][8];
+  u32x4 qf[2][4];      // B fragments of the query tiles
+  const uint8_t *ring;
+  int kofs[4], vofs[4];  // the lane's fragments within a ring slot
+
+  // Ring slot: 32 rows of K, then 32 of V, in 1 KB groups of whole rows (4;
+  // FP8 8), so that one load instruction covers whole rows (18 cycles of the
+  // CU's load path; 64 where each lane reads another row).  Within a group
+  // the 16-byte units of row r are permuted (BF16: unit u at u ^ 4 (r & 3);
+  // FP8: u ^ 2 ((r >> 1) & 3)) and the groups are padded, so that the fragment
+  // reads below fall on different banks.
+  static constexpr int kRowBytes = FP8 ? 128 : 256;
+  static constexpr int kUnits = kRowBytes / 16;
+  static constexpr int kGroupRows = 1024 / kRowBytes;
+  static constexpr int kGroups = 32 / kGroupRows;  // of each of K and V
+  static constexpr int kKGroup = 1040;             // group stride of K
+  static constexpr int kVGroup = 1056;             // group stride of V (BF16)
+  static constexpr int kKBytes = kGroups * kKGroup;
+  static constexpr int kSlotBytes = kKBytes + (FP8 ? kGroups * 1024 + 32 : kGroups * kVGroup);
+  // Byte offset of V's group g from the slot's start (FP8: 16 bytes of padding per 16 rows).
+  static constexpr int v_group(int g) { return kKBytes + (FP8 ? g * 1024 + (g >> 1) * 16 : g * kVGroup); }
+  // Two workgroups of four waves per CU, or one of eight: four slots where
+  // one group shares the ring, two for each of several groups.
+  static constexpr int kSlots = NW;
+  // 1 KB loads per wave and block: waves 0 .. NW / 2 - 1 load K, the others V.
+  static constexpr int kLoads = 2 * kGroups / NW;
+
+  static __device__ __forceinline__ int swizzle(int r) { return FP8 ? (r & 6) : 4 * (r & 3); }
+
+  __device__ __forceinline__ void reset(const uint8_t *group_ring) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      nmax[t] = INFINITY;
+      lsum[t] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    ring = group_ring;
+    // K: row col of a 16-row block.  BF16: 8 dims 32c + 8 quad .. (unit 4c +
+    // quad).  FP8: 16 dims 64j + 16 quad .. (unit 4j + quad), which the query
+    // fragments 2j and 2j + 1 hold in the same order.
+    const int kr = (col / kGroupRows) * kKGroup + (col % kGroupRows) * kRowBytes;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) kofs[c] = kr + ((4 * (FP8 ? c & 1 : c) + quad) ^ swizzle(col)) * 16;
+    // Vᵀ, dims 16 e .. 16 e + 15, tokens 4 quad + [0, 4) of both 16-row blocks
+    // in the order of the Pᵀ fragment, e = 2x + y (y: an immediate offset).
+    // BF16 (ds_read_b64_tr_b16, one read per 16-row block: within 16 lanes,
+    // lane i receives element i % 4 of the 8 bytes lane 4k + i / 4 addresses, k
+    // = 0..3): lane i addresses dims 16 e + 4 (i % 4) .. of token row 4 quad +
+    // i / 4.  FP8 (ds_read_b64_tr_b8, one read: lane i receives byte i % 8 of
+    // the 8 bytes lane 2k + i / 8 addresses, k = 0..7): lane i addresses dims
+    // 16 e + 8 (i & 1) .. of token row 4 quad + (i >> 1) % 4 of block i >> 3.
+    const int i = col;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      if constexpr (FP8) {
+        const int r = 4 * quad + ((i >> 1) & 3), g = 2 * (i >> 3) + (r >> 3);
+        vofs[x] = v_group(g) + (r & 7) * 128 + (2 * x ^ swizzle(r)) * 16 + 8 * (i & 1);
+      } else {
+        vofs[x] = v_group(quad) + (i >> 2) * 256 + ((4 * x ^ swizzle(i >> 2)) + ((i & 3) >> 1)) * 16 +
+                  8 * (i & 1);
+      }
+    }
+  }
+
+  // Query fragment c: B fragment of S (lane: column, k = 8 quad + [0, 8)).
+  static __device__ __forceinline__ int q_dim(int c, int quad) {
+    return FP8 ? 64 * (c >> 1) + 16 * quad + 8 * (c & 1) : 32 * c + 8 * quad;
+  }
+
+  // K fragments of a block (A fragments of S: token row, k as above), by
+  // chunk and 16-row block.
+  struct KFrags {
+    u32x4 f[FP8 ? 2 : 4][2];
+  };
+  __device__ __forceinline__ KFrags read_k(int slot) const {
+    KFrags k;
+#pragma unroll
+    for (int c = 0; c < (FP8 ? 2 : 4); ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        k.f[c][h] = *reinterpret_cast<const u32x4 *>(ring + kofs[c] + slot + h * (kGroups / 2) * kKGroup);
+    return k;
+  }
+  // Scores of a block: s[t][h][i] = S[token 16 h + 4 quad + i][column of tile t].
+  struct Scores {
+    f32x4 s[2][2];
+    __device__ __forceinline__ float get(int x) const { return s[x >> 3][(x >> 2) & 1][x & 3]; }
+  };
+  // S = K·Qᵀ, product x of 8: chunk x >> 1, 16-row block x & 1, both tiles.
+  __device__ __forceinline__ void score(const KFrags &k, Scores &sc, int x) const {
+    const int c = x >> 1, h = x & 1;
+    const u32x4 w = FP8 ? fp8x8_to_bf16x8(u32x2{k.f[c >> 1][h][2 * (c & 1)], k.f[c >> 1][h][2 * (c & 1) + 1]})
+                        : k.f[FP8 ? 0 : c][h];
+    const f32x4 z = {};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      sc.s[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w), as_bf16x8(qf[t][c]),
+                                                           c ? sc.s[t][h] : z, 0, 0, 0);
+  }
+
+  // Vᵀ fragments of a block, by 16-dim block.
+  struct VFrags {
+    u32x4 f[8];
+  };
+  __device__ __forceinline__ u32x4 read_v(int slot, int e) const {
+    const uint8_t *p = ring + vofs[e >> 1] + slot + (e & 1) * (FP8 ? 16 : 32);
+    if constexpr (FP8) {
+      const u32x2 b = lds_read_tr8(p);
+      return u32x4{b[0], b[1], 0, 0};
+    } else {
+      const u32x2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + (v_group(4) - v_group(0)));
+      return u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
+  }
+
+  // Weights as B fragments of the product (lane: column, k = 8 quad + j is
+  // token 16 (j >> 2) + 4 quad + (j & 3)), and their residuals.
+  struct Weights {
+    u32x4 hi[2], lo[2];
+  };
+  // O += P·V, dims 16 e .. of both tiles.
+  __device__ __forceinline__ void product(const VFrags &v, const Weights &p, int e) {
+    const bf16x8 w = as_bf16x8(FP8 ? fp8x8_to_bf16x8(u32x2{v.f[e][0], v.f[e][1]}) : v.f[e]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, as_bf16x8(p.hi[t]), acc[t][e], 0, 0, 0);
+    if constexpr (HL)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, as_bf16x8(p.lo[t]), acc[t][e], 0, 0, 0);
+  }
+
+  // Weights 2y, 2y + 1 of the lane's 16 (already exponentiated; 8 per tile)
+  // into the fragments, and into the normalizer l of the tile.
+  static __device__ __forceinline__ void put(Weights &p, float &l, float x0, float x1, int y) {
+    if constexpr (HL) {
+      const uint32_t b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
+      p.hi[y >> 2][y & 3] = pack_hi16(b0, b1);
+      p.lo[y >> 2][y & 3] = pack_hi16(__float_as_uint(x0 - __uint_as_float(b0 & 0xffff0000u)),
+                                      __float_as_uint(x1 - __uint_as_float(b1 & 0xffff0000u)));
+      l += x0;
+      l += x1;
+    } else {
+      const uint32_t w = bf16x2_pack(x0, x1);
+      p.hi[y >> 2][y & 3] = w;
+      typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+      l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w),
+                                          __builtin_bit_cast(bf16x2, 0x3F803F80u), l, false);
+    }
+  }
+
+  // Holds the values' computation at this place of the instruction stream.
+  static __device__ __forceinline__ void pin(f32x4 &m, f32x4 &n, float &x, float &y, float &z) {
+    asm volatile("" : "+v"(m), "+v"(n), "+v"(x), "+v"(y), "+v"(z));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // Masks the scores of tokens at or past a column's causal end (lt0: the
+  // block's first token).
+  __device__ __forceinline__ void mask(Scores &cur, int64_t lt0) const {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int vis = (int)max<int64_t>(-1, min<int64_t>(32, end_col[t] - lt0));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        cur.s[t][0][i] = (quad * 4 + i < vis) ? cur.s[t][0][i] : -INFINITY;
+        cur.s[t][1][i] = (16 + quad * 4 + i < vis) ? cur.s[t][1][i] : -INFINITY;
+      }
+    }
+  }
+
+  // One step of the software pipeline, block j of the wave's group:
+  //   products of block j - 1 (v, w)    |  scaling and half the exponentials
+  //   scores of block j + 1             |  the rest of block j's softmax, and
+  //                                     |  the reads of block j's V
+  // `cur`: block j's scores; on return `nxt` holds block j + 1's, v and w
+  // block j's.  kslot, vslot: ring offsets of K (j + 1) and V (j).  (After
+  // the last block the scores of whatever K's slot holds are not used.)
+  __device__ __forceinline__ void step(int kslot, int vslot, Scores &cur, Scores &nxt, VFrags &v,
+                                       Weights &w) {
+    const KFrags k = read_k(kslot);
+    float p[16];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      product(v, w, x);
+      p[2 * x] = fmaf(cur.get(2 * x), a.scale_log2, nmax[x >> 2]);
+      p[2 * x + 1] = fmaf(cur.get(2 * x + 1), a.scale_log2, nmax[x >> 2]);
+      if (x > 0) p[x - 1] = fast_exp2(p[x - 1]);
+      pin(acc[0][x], acc[1][x], p[2 * x], p[2 * x + 1], p[x > 0 ? x - 1 : 0]);
+    }
+    Weights wn;
+    float l[2] = {lsum[0], lsum[1]};
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      score(k, nxt, x);
+      if (x < 5) {
+        p[2 * x + 7] = fast_exp2(p[2 * x + 7]);
+        if (x < 4) p[2 * x + 8] = fast_exp2(p[2 * x + 8]);
+      }
+      if (x < 7) put(wn, l[x >> 2], p[2 * x], p[2 * x + 1], x);
+      if (x == 6) put(wn, l[1], p[14], p[15], 7);
+      v.f[x] = read_v(vslot, x);
+      pin(nxt.s[0][x & 1], nxt.s[1][x & 1], l[x >> 2], p[x < 5 ? 2 * x + 7 : 15],
+          p[x < 4 ? 2 * x + 8 : 15]);
+    }
+    // The reference max of a column moves only when its normalizer passes
+    // kRefreshNormalizer or is not a number (no reference yet, or an
+    // overflow): BF16 and FP32 weights keep their relative precision at any
+    // magnitude, so a reference below the running max costs none, and the
+    // common step needs no max at all.  LSE = reference max + log2(normalizer).
+    if (__builtin_amdgcn_ballot_w64(!(l[0] <= kRefreshNormalizer && l[1] <= kRefreshNormalizer))) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float mx = fmaxf(cur.get(8 * t), cur.get(8 * t + 1));
+#pragma unroll
+        for (int i = 2; i < 8; ++i) mx = fmaxf(mx, cur.get(8 * t + i));
+        mx = quad_max(mx) * a.scale_log2;
+        const float m_old = -nmax[t];
+        const float m_new = fmaxf(m_old, mx);
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new;  // nothing visible yet
+        // (a column with nothing visible before has O = 0: nothing to rescale)
+        const float al = fast_exp2(m_old - m_use);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[t][e] *= al;
+        nmax[t] = -m_new;
+        l[t] = lsum[t] * al;
+#pragma unroll
+        for (int y = 4 * t; y < 4 * t + 4; ++y)
+          put(wn, l[t], fast_exp2(fmaf(cur.get(2 * y), a.scale_log2, -m_use)),
+              fast_exp2(fmaf(cur.get(2 * y + 1), a.scale_log2, -m_use)), y);
+      }
+    }
+    lsum[0] = l[0];
+    lsum[1] = l[1];
+    w = wn;
+  }
+
+  // The whole causal walk of the wave's group over 16-row blocks 0..n16-1 (the
+  // second half of the last 32-token block is empty when n16 is odd: no rows).
+  // load(b, slot): the wave's share of block b to the slot at LDS address
+  // `slot` (blocks past the end: no rows, zeros).  `loads_k`: the wave loads K
+  // rows, else V rows; K runs one block ahead of V, so that one barrier per
+  // step publishes K (j + 1) and V (j), the loads of the next kSlots - 1 steps
+  // are in flight, and a slot is refilled one step after it was read.
+  // first(): called once the first loads are out.
+  template <class Load, class First>
+  __device__ __forceinline__ void stream(int n16, Load load, First first, uint32_t lds, bool loads_k, int grp,
+                                         int64_t own_end) {
+    const int nb = (n16 + 1) >> 1;
+    const int steps = (nb + G - 1) / G;
+    // this group's blocks that the wave computes, and the blocks (of all
+    // groups) that need no mask
+    const int nbw = uni(max(0, ((int)min<int64_t>((own_end + 31) >> 5, nb) - grp + G - 1) / G));
+    const int nfull = uni((int)min<int64_t>(full_end >> 5, nb));
+    // (K) block j + kSlots goes to the slot of block j, (V) one less
+    const int ahead = uni(kSlots - (loads_k ? 0 : 1));
+    auto slot_of = [](int j) { return (j & (kSlots - 1)) * kSlotBytes; };
+    if (loads_k) load(grp, lds);
+#pragma unroll
+    for (int j = 1 - kSlots; j < 0; ++j)
+      load(G * (j + ahead) + grp, lds + slot_of(j + ahead));
+    first();
+    publish<(kSlots - 1) * kLoads>();
+    // (s: j, or its slot)
+    auto advance = [&](int j, int s) {
+      publish<(kSlots - 2) * kLoads>();
+      load(G * (j + ahead) + grp, lds + slot_of(s + ahead));
+    };
+    Scores sa, sb;
+    VFrags v = {};
+    Weights w = {};
+    if (nbw > 0) {
+      const KFrags k = read_k(0);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) score(k, sa, c);
+    }
+    int j = 0;
+    while (j < nbw) {
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        if (s > 0 && j >= nbw) break;
+        advance(j, s);
+        Scores &cur = s & 1 ? sb : sa, &nxt = s & 1 ? sa : sb;
+        if (G * j + grp >= nfull) mask(cur, 32 * (int64_t)(G * j + grp));
+        step(slot_of(s + 1), slot_of(s), cur, nxt, v, w);
+        ++j;
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 8; ++x) product(v, w, x);
+    for (; j < steps; ++j) advance(j, j);
+    wait_vmcnt<0>();
+  }
+
+  // Waits until at most N of this wave's loads are outstanding (and for its
+  // LDS reads, so that a slot read before the barrier may be refilled after
+  // it), then meets the workgroup's other waves.
+  template <int N>
+  static __device__ __forceinline__ void publish() {
+    static_assert(N < 64, "vmcnt field");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(((N >> 4) << 14) | (0x0 << 8) | (0x7 << 4) | (N & 15));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+};
+
 // Query tiles per wave of the long-tile algorithm: two (128 columns per
 // workgroup) when that still gives at least kLongTwoMinGrid workgroups (two
 // per CU), else one (64 columns).  Measured on GQA4 32/8 prompts, two tiles
@@ -651,173 +1230,23 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, quad = lane >> 4;
-  const int kvh = (int)(blockIdx.x % a.hkv);
-  // Tiles in reverse order: a request's later rows see longer causal ranges,
-  // so the heaviest tiles are dispatched first and the launch does not end
-  // with a few long tiles running alone (the grid's excess workgroups, which
-  // find no tile, come first and exit at once).  Workgroup b runs on XCD
-  // b % 8; with the kv-head fastest, each XCD keeps to a fixed set of
-  // kv-heads, whose K/V its L2 shares across tiles.
-  const int64_t n_tiles = (int64_t)(gridDim.x / a.hkv), m = blockIdx.x / a.hkv;
-  int64_t rank = m;
-  if (a.tile_layer > 0) {
-    // Serpentine: every other layer of tile_layer workgroups (one per CU of
-    // the XCDs this kv-head runs on) takes its tiles in reverse, so a CU's
-    // successive workgroups pair heavy tiles with light ones instead of
-    // stacking the heaviest of every layer.
-    const int64_t L = a.tile_layer, layer = m / L, c = m - layer * L;
-    const int64_t width = min(L, n_tiles - layer * L);
-    rank = layer * L + ((layer & 1) ? width - 1 - c : c);
-  }
-  const int64_t tile = n_tiles - 1 - rank;
-  const bool interleave = !RAGGED && LT && a.tile_interleave != 0;
-
-  // Metadata in as few dependent round trips as possible: the global guard
-  // words and every request's qo range, page (kv) range and tail are loaded
-  // together; the guards are applied after the scan that locates this tile.
-  const int32_t qo0 = a.qo[0], qoB = a.qo[a.batch];
-  const int32_t ip0 = a.indptr[0], ipB = a.indptr[a.batch];
   // A page-index array of at most 128 entries (the reference's shapes) is
-  // loaded whole in the same round trip, two words per lane: the request's
-  // page indices and their check then come from registers, so the query tile
-  // and the first K/V blocks share the second round trip.
+  // loaded whole with the metadata, two words per lane: the request's page
+  // indices and their check then come from registers, so the query tile and
+  // the first K/V blocks share the second round trip.
   const bool small_table = !RAGGED && !SH && a.n_indices <= 128;
   int tbl0 = 0, tbl1 = 0;
   if (small_table) {
     if (lane < a.n_indices) tbl0 = a.indices[lane];
     if (lane + 64 < a.n_indices) tbl1 = a.indices[lane + 64];
   }
-
-  // Locate the request owning this tile: prefix of the requests' tile counts.
-  // Paged (prefill.rs:303-313): rows belong to the requests before the first
-  // malformed qo range.  Ragged (prefill.rs:111-137): row q belongs to the
-  // first request r with q < qo_indptr[r+1], i.e. r owns the rows from
-  // max(qo_indptr[r], max(qo_indptr[1..r])) to qo_indptr[r+1], and a request
-  // failing its guards keeps its rows' sentinels.
-  if (tid == 0) sm.req = -1;
-  int64_t carry = 0;
-  int32_t carry_max = 0;
-  for (int base = 0; base < a.batch; base += W * 64) {
-    const int r = base + tid;
-    int64_t cnt = 0;
-    int32_t s0 = 0, s1 = 0, p0 = 0, p1 = 0, t1 = 0, fbeg = 0;
-    if (r < a.batch) {
-      s0 = a.qo[r];
-      s1 = a.qo[r + 1];
-      p0 = a.indptr[r];
-      p1 = a.indptr[r + 1];
-      if constexpr (!RAGGED) t1 = a.last[r];
-    }
-    if constexpr (RAGGED) {
-      // exclusive running max of the qo ends before r
-      int32_t x = r < a.batch ? s1 : INT32_MIN;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x = max(x, y);
-      }
-      if (lane == 63) sm.wave_max[wave] = x;
-      __syncthreads();
-      int32_t before = carry_max, blk = carry_max;
-#pragma unroll
-      for (int i = 0; i < W; ++i) {
-        before = i < wave ? max(before, sm.wave_max[i]) : before;
-        blk = max(blk, sm.wave_max[i]);
-      }
-      const int32_t up = __shfl_up(x, 1, 64);
-      const int32_t excl = lane > 0 ? max(before, up) : before;
-      carry_max = blk;
-      if (r < a.batch) {
-        const bool ok = s0 >= 0 && s1 > s0 && s1 <= a.nnz && p0 >= 0 && p1 > p0 &&
-                        p1 <= a.nnz_kv && s1 - s0 <= p1 - p0;
-        const int32_t lo = max(s0, excl);
-        if (ok && s1 > lo) {
-          cnt = ((int64_t)(s1 - lo) * a.group + TC - 1) / TC;
-          fbeg = (lo - s0) * a.group;
-        }
-      }
-    } else {
-      if (r < a.batch)
-        cnt = (s0 >= 0 && s1 > s0 && s1 <= a.nnz) ? ((int64_t)(s1 - s0) * a.group + TC - 1) / TC
-                                                  : kNoTiles;
-    }
-    if (interleave && wave == 0) {
-      // (at most 64 requests: wave 0 holds every count, one pass.)  Rank
-      // rank - excess is the j-th of the tiles k from their request's end,
-      // where k is the largest with F(k) = sum of min(k, count) <= it and j
-      // counts requests with more than k tiles in request order; requests
-      // from the first malformed qo range on own no tile.
-      const bool in = r < a.batch;
-      const uint64_t badm = __ballot(in && cnt == kNoTiles);
-      const int first_bad = badm ? __builtin_ctzll(badm) : 64;
-      const int c = (in && lane < first_bad) ? (int)cnt : 0;
-      const int total = wave_sum_i32(c);
-      const int64_t rr = rank - (n_tiles - total);
-      if (rr >= 0) {
-        int lo = 0, hi = wave_max_i32(c);
-        while (hi - lo > 1) {
-          const int mid = (lo + hi) >> 1;
-          if (wave_sum_i32(min(mid, c)) <= rr) lo = mid;
-          else hi = mid;
-        }
-        const int j = (int)(rr - wave_sum_i32(min(lo, c)));
-        const uint64_t more = __ballot(c > lo);
-        const int below = (int)__builtin_amdgcn_mbcnt_hi(
-            (uint32_t)(more >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)more, 0u));
-        if (c > lo && below == j) {
-          sm.req = r;
-          sm.tile0 = c - 1 - lo;
-          sm.meta[0] = s0;
-          sm.meta[1] = s1;
-          sm.meta[2] = p0;
-          sm.meta[3] = p1;
-          sm.meta[4] = t1;
-          sm.meta[5] = fbeg;
-        }
-      }
-    }
-    const int64_t x = wave_incl_scan64(cnt, lane);
-    if (lane == 63) sm.wave_tot[wave] = x;
-    __syncthreads();
-    int64_t before = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < W; ++i) {
-      const int64_t t = sm.wave_tot[i];
-      before += (i < wave) ? t : 0;
-      tot += t;
-    }
-    const int64_t incl = carry + before + x;
-    if (!interleave && r < a.batch && tile < incl && tile >= incl - cnt && cnt != kNoTiles) {
-      sm.req = r;
-      sm.tile0 = (int32_t)(tile - (incl - cnt));
-      sm.meta[0] = s0;
-      sm.meta[1] = s1;
-      sm.meta[2] = p0;
-      sm.meta[3] = p1;
-      sm.meta[4] = t1;
-      sm.meta[5] = fbeg;
-    }
-    carry += tot;
-    __syncthreads();
-    if (carry > tile || interleave) break;
-  }
-  // Global guards (prefill.rs:293-300 paged, :102-108 ragged).
-  if constexpr (RAGGED) {
-    if (qo0 != 0 || qoB != a.nnz || ip0 != 0 || ipB != a.nnz_kv) return;
-  } else {
-    const bool pages_ok = ipB >= 0 && (a.indices_capacity ? (int64_t)ipB <= a.n_indices
-                                                          : (int64_t)ipB == a.n_indices);
-    if (qo0 != 0 || qoB != a.nnz || ip0 != 0 || !pages_ok) return;
-  }
-  const int r = uni(sm.req);
-  if (r < 0) return;
-  const int tile0 = uni(sm.tile0);
-  const int fbeg = uni(sm.meta[5]);
+  TileLoc loc;
+  if (!locate_tile<W, RAGGED, TC, LT != 0>(a, sm.loc, loc)) return;
+  const int kvh = loc.kvh, tile0 = loc.tile0;
+  const int32_t fbeg = loc.fbeg, qs = loc.qs, qe = loc.qe, ps = loc.ps, pe = loc.pe;
 
   // Per-request guards (paged: prefill.rs:316-342; ragged: applied in the
   // scan above, a failing request owns no tile).
-  const int32_t qs = uni(sm.meta[0]), qe = uni(sm.meta[1]);
-  const int32_t ps = uni(sm.meta[2]), pe = uni(sm.meta[3]);
   int req_pages;
   int32_t tl;
   int64_t kv_len;
@@ -826,8 +1255,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     req_pages = (int)((kv_len + 15) / 16);
     tl = (int32_t)(kv_len - (int64_t)(req_pages - 1) * 16);
   } else {
-    tl = uni(sm.meta[4]);
-    if (ps < 0 || pe <= ps || pe > ipB || tl < 1 || tl > a.page_rows) return;
+    tl = loc.tl;
+    if (ps < 0 || pe <= ps || pe > loc.ipB || tl < 1 || tl > a.page_rows) return;
     kv_len = (int64_t)(pe - ps - 1) * a.page_rows + tl;
     // 16-row blocks of the request and the valid rows of its last one
     req_pages = (int)((kv_len + 15) / 16);
@@ -1134,6 +1563,281 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
   if (quad == 0) a.lse[row_head] = M + __log2f(L);
 }
 
+// The pipelined long-tile kernels: paged (BF16 or FP8 pages, weights rounded
+// to BF16) and ragged (HL: weights as high part and residual, as the ragged
+// contract's other algorithms keep them).
+template <int W, int NW>
+struct PipeSmem {
+  LocateSmem<W> loc;
+  float m[W][32], l[W][32];  // the groups' column states
+  uint32_t bad[W];
+  int32_t next_idx[W][64];   // next window's page indices (paged)
+};
+
+template <int W, int NW, bool RAGGED, bool FP8>
+__device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
+  constexpr int G = W / NW;
+  constexpr int TC = 32 * NW;  // flattened columns per workgroup
+  using Wave = PipeWave<NW, FP8, RAGGED, G>;
+  // FP8 pages: K's scale folds into the score scale, V's into the output.
+  PrefillArgs a = args;
+  float v_scale = 1.0f;
+  if constexpr (FP8) {
+    a.scale_log2 *= a.kv_scales[0];
+    v_scale = a.kv_scales[1];
+  }
+  __shared__ PipeSmem<W, NW> sm;
+  // the groups' rings (several groups: also the merge staging of their column
+  // states, 64 floats per lane)
+  constexpr int kRingBytes = G * Wave::kSlots * Wave::kSlotBytes;
+  constexpr int kMergeBytes = G > 1 ? W * 64 * 64 * 4 : 0;
+  __shared__ __align__(16) uint8_t lring[kRingBytes > kMergeBytes ? kRingBytes : kMergeBytes];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, quad = lane >> 4;
+  TileLoc loc;
+  if (!locate_tile<W, RAGGED, TC, true>(a, sm.loc, loc)) return;
+  const int kvh = loc.kvh;
+  const int32_t qs = loc.qs, ps = loc.ps, pe = loc.pe;
+  // Per-request guards (paged: prefill.rs:316-342; ragged: applied by the
+  // search, a failing request owns no tile).
+  int64_t kv_len;
+  if constexpr (RAGGED) {
+    kv_len = pe - ps;
+  } else {
+    if (ps < 0 || pe <= ps || pe > loc.ipB || loc.tl < 1 || loc.tl > a.page_rows) return;
+    kv_len = (int64_t)(pe - ps - 1) * a.page_rows + loc.tl;
+  }
+  // 16-row blocks of the request and the valid rows of its last one
+  const int req_pages = (int)((kv_len + 15) / 16);
+  const int tl = (int)(kv_len - (int64_t)(req_pages - 1) * 16);
+  const int qo_len = loc.qe - qs;
+  if ((int64_t)qo_len > kv_len) return;
+
+  // (fcols <= nnz_qo * Hq fits int32: the plan checks it)
+  const int fcols = qo_len * a.group, col0 = loc.fbeg + loc.tile0 * TC;
+  auto row_of = [&](int f) { return (int)((uint32_t)f / (uint32_t)a.group); };
+  const int wq = wave % NW, grp = wave / NW;  // the wave's tiles and its group
+  const int own0 = col0 + 32 * wq;
+  // the tile's causal page range (16-row blocks, up to its last column's end)
+  const int npages =
+      uni((int)((kv_len - qo_len + row_of(min(col0 + TC - 1, fcols - 1)) + 1 + 15) / 16));
+  // this lane's column of each of the wave's tiles
+  Wave lw{a, lane, col, quad};
+  bool colv_t[2];
+  int qi_t[2], gh_t[2];
+  {
+    // the smallest causal end of the wave's valid columns: blocks before it
+    // need no mask (the columns past fcols are discarded, so they do not count)
+    int64_t fe = INT64_MAX;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int ft = own0 + 16 * t + col;
+      colv_t[t] = ft < fcols;
+      qi_t[t] = colv_t[t] ? row_of(ft) : 0;
+      gh_t[t] = colv_t[t] ? ft - qi_t[t] * a.group : 0;
+      lw.end_col[t] = colv_t[t] ? kv_len - qo_len + qi_t[t] + 1 : 0;
+      fe = colv_t[t] ? min(fe, lw.end_col[t]) : fe;
+    }
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) {
+      const int64_t y = ((int64_t)__shfl_xor((int)(fe >> 32), o, 64) << 32) |
+                        (uint32_t)__shfl_xor((int)(uint32_t)fe, o, 64);
+      fe = min(fe, y);
+    }
+    lw.full_end = uni64(fe);
+    lw.reset(lring + grp * Wave::kSlots * Wave::kSlotBytes);
+  }
+  // The first window of page indices, then the query tiles: the first K/V
+  // loads wait for the former only.
+  int idx = 0;
+  if constexpr (!RAGGED) idx = lane < npages ? a.indices[ps + (lane >> a.blocks_lg)] : 0;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const uint16_t *qp = colv_t[t] ? a.q + ((int64_t)(qs + qi_t[t]) * a.hq +
+                                            (int64_t)kvh * a.group + gh_t[t]) * 128
+                                   : a.q;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) lw.qf[t][c] = load16(qp + Wave::q_dim(c, quad));
+  }
+  // The wave's loads of 32-token block b straight into LDS
+  // (PipeWave::stream).  Lane l holds the address and the valid bytes of
+  // 16-row block 64 win + l of its matrix (K or V), computed once per 64
+  // blocks; the next window's page indices are in flight meanwhile.  An index
+  // failing the guard has no valid bytes, so its loads read zeros, as do rows
+  // past a page's valid rows.
+  constexpr int kElem = FP8 ? 1 : 2;
+  const bool loads_k = wq < NW / 2;
+  const int row_bytes = a.row_elems * kElem;
+  const uint64_t kv_base = (uint64_t)(loads_k ? a.k : a.v) + (int64_t)kvh * a.head_elems * kElem;
+  // The next window's page indices go to LDS as the blocks do (a load into a
+  // register would make the compiler wait for every load in flight), and are
+  // read back when the window starts, many steps later.
+  int win = -1;
+  uint32_t blk_lo = 0, blk_hi = 0;
+  int blk_bytes = 0;
+  int lane_off[4] = {0, 0, 0, 0};  // this lane's byte offset within each load of a 16-row block
+  {
+    const int sub = (lane & (Wave::kUnits - 1)) ^ Wave::swizzle(lane / Wave::kUnits);
+#pragma unroll
+    for (int x = 0; x < 16 / Wave::kGroupRows; ++x)
+      lane_off[x] = (x * Wave::kGroupRows + lane / Wave::kUnits) * row_bytes + sub * 16;
+  }
+  auto load_block = [&](int b, uint32_t slot) {
+    if ((b >> 5) != win) {
+      win = b >> 5;
+      const int x = 64 * win + lane;
+      int rows = x < npages ? (x == req_pages - 1 ? tl : 16) : 0;
+      uint64_t at;
+      if constexpr (RAGGED) {
+        at = kv_base + ((uint64_t)ps + (uint64_t)x * 16) * (uint64_t)row_bytes;
+      } else {
+        const int pg = win == 0 ? idx : sm.next_idx[wave][lane];
+        if (pg < 0 || (int64_t)pg >= a.pool) rows = 0;
+        at = kv_base + (uint64_t)(uint32_t)pg * (uint32_t)(a.page_rows * a.hkv * 128 * kElem) +
+             (uint32_t)(x & ((1 << a.blocks_lg) - 1)) * (uint32_t)(16 * row_bytes);
+      }
+      blk_lo = (uint32_t)at;
+      blk_hi = (uint32_t)(at >> 32);
+      blk_bytes = rows > 0 ? ((rows - 1) * a.row_elems + 128) * kElem : 0;
+      if constexpr (!RAGGED) {
+        asm volatile("" ::"v"(blk_lo), "v"(blk_hi), "v"(blk_bytes) : "memory");  // next_idx is read
+        const int64_t first = ((int64_t)(win + 1) * 64) >> a.blocks_lg;
+        const int n = (int)max<int64_t>(0, min<int64_t>(64, (int64_t)(pe - ps) - first));
+        lds_load4(__builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t *>(a.indices + ps + first), 0,
+                                                    4 * n, 0x00020000),
+                  &sm.next_idx[wave][0], (lane >> a.blocks_lg) * 4);
+      }
+    }
+#pragma unroll
+    for (int y = 0; y < (NW == 4 ? 1 : 2); ++y) {
+      const int h = NW == 4 ? (wq & 1) : y;
+      const int l = (2 * b + h) & 63;
+      const uint64_t at = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)blk_hi, l) << 32) |
+                          (uint32_t)__builtin_amdgcn_readlane((int)blk_lo, l);
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<void *>(at), 0, __builtin_amdgcn_readlane(blk_bytes, l), 0x00020000);
+      constexpr int kHalf = Wave::kGroups / 2;
+#pragma unroll
+      for (int x = 0; x < kHalf; ++x) {
+        const uint32_t kg = (uint32_t)((h * kHalf + x) * Wave::kKGroup);
+        const uint32_t vg = (uint32_t)(Wave::v_group(x) + h * (Wave::v_group(kHalf) - Wave::v_group(0)));
+        lds_load16_at(r, slot + (loads_k ? kg : vg), lane_off[x]);
+      }
+    }
+  };
+  // causal end of this wave's last column (0: the wave's tile is empty)
+  const int64_t own_end =
+      own0 < fcols
+          ? kv_len - qo_len + row_of(min(own0 + 31, fcols - 1)) + 1
+          : 0;
+  const uint32_t ring_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lring +
+                            (uint32_t)(grp * Wave::kSlots * Wave::kSlotBytes);
+  // While the first blocks are on their way: every page index of the request
+  // is checked (the reference rejects the whole request; the verdict is read
+  // after the walk), and the columns past the tile's last get zero queries.
+  bool bad = false;
+  auto mask_q = [&]() {
+    if constexpr (!RAGGED)
+      for (int i = tid; i < pe - ps; i += W * 64) {
+        const int32_t x = a.indices[ps + i];
+        bad |= x < 0 || (int64_t)x >= a.pool;
+      }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) lw.qf[t][c] = colv_t[t] ? lw.qf[t][c] : u32x4{0, 0, 0, 0};
+  };
+  lw.stream(npages, load_block, mask_q, ring_lds, loads_k, grp, uni64(own_end));
+
+  // Each wave finishes its own tiles; an invalid page index anywhere in the
+  // request keeps its sentinels.
+  float L[2], M[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    L[t] = quad_sum(lw.lsum[t]);
+    M[t] = -lw.nmax[t];
+    if (G > 1 && quad == 0) {
+      sm.m[wave][16 * t + col] = M[t];
+      sm.l[wave][16 * t + col] = L[t];
+    }
+  }
+  if (block_or(bad, sm.bad)) return;
+  constexpr int kOwn = 8 / G;  // 16-dim blocks that a group finishes
+  if constexpr (G > 1) {
+    // The groups' states merge as split-K states do: every wave writes the
+    // dims that other groups finish to the ring's LDS (all waves are past
+    // their last ring read: block_or's barrier), and group g finishes dims
+    // 128 g / G .. of its columns.
+    f32x4 *xs = reinterpret_cast<f32x4 *>(lring) + lane;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e / kOwn != grp) xs[((wave * 2 + t) * 8 + e) * 64] = lw.acc[t][e];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) M[t] = fmaxf(M[t], sm.m[g * NW + wq][16 * t + col]);
+      float f[G];
+      L[t] = 0.0f;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const float m = sm.m[g * NW + wq][16 * t + col];
+        f[g] = m == -INFINITY ? 0.0f : fast_exp2(m - M[t]);
+        L[t] = fmaf(sm.l[g * NW + wq][16 * t + col], f[g], L[t]);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (e / kOwn != grp) continue;
+        f32x4 o = {};
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const f32x4 x = g == grp ? lw.acc[t][e] : xs[(((g * NW + wq) * 2 + t) * 8 + e) * 64];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = fmaf(x[i], f[g], o[i]);
+        }
+        lw.acc[t][e] = o;
+      }
+    }
+  }
+  // O through LDS (the ring is free; several groups: past a second barrier,
+  // since other waves may still read the merge staging), each wave its own 32
+  // rows of 256 bytes at a stride of 272: whole rows then go out 16 bytes per
+  // lane (18 cycles of the CU's store path per KB; 8-byte pieces of 16 rows
+  // per instruction took 64, 2 us per workgroup of four waves).
+  if constexpr (G > 1) __syncthreads();
+  uint8_t *ot = lring + wave * 32 * 272;
+  int row_head[2];  // output row of each tile's column, -1: none
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const float inv = 1.0f / L[t];
+    row_head[t] = colv_t[t] ? (qs + qi_t[t]) * a.hq + kvh * a.group + gh_t[t] : -1;
+    // acc[t][e][i] = O[column][16 e + 4 quad + i]
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (e / kOwn == grp)
+        *reinterpret_cast<u32x2 *>(ot + (16 * t + col) * 272 + 32 * e + 8 * quad) =
+            u32x2{bf16x2_pack(lw.acc[t][e][0] * inv * v_scale, lw.acc[t][e][1] * inv * v_scale),
+                  bf16x2_pack(lw.acc[t][e][2] * inv * v_scale, lw.acc[t][e][3] * inv * v_scale)};
+    if (quad == 0 && grp == 0 && colv_t[t]) a.lse[row_head[t]] = M[t] + __log2f(L[t]);
+  }
+  wave_lds_fence();
+  // the group's 16-byte units of each row
+  constexpr int kOwnUnits = 2 * kOwn, kRowsPer = 64 / kOwnUnits;
+  const int unit = grp * kOwnUnits + (lane & (kOwnUnits - 1));
+#pragma unroll
+  for (int x = 0; x < 32 / kRowsPer; ++x) {
+    const int r = x * kRowsPer + lane / kOwnUnits;  // column of the wave
+    const int rh0 = __shfl(row_head[0], r & 15, 64), rh1 = __shfl(row_head[1], r & 15, 64);
+    const int rh = r < 16 ? rh0 : rh1;
+    if (rh >= 0)
+      *reinterpret_cast<u32x4 *>(a.out + (int64_t)rh * 128 + unit * 8) =
+          *reinterpret_cast<const u32x4 *>(ot + r * 272 + unit * 16);
+  }
+}
+
 // At least three waves per SIMD: the per-block chain (MFMA, softmax, MFMA)
 // leaves a wave waiting most of the time, and a third wave per SIMD fills
 // those gaps (the four-wave BF16 kernel would otherwise settle at two).
@@ -1147,6 +1851,13 @@ constexpr int kPrefillWavesPerEu = 3;
 template <int W, bool FP8, bool SH = false, int LT = 0>
 __global__ __launch_bounds__(W * 64, LT ? (W == 8 ? (LT == 1 ? 4 : 2) : 3) : kPrefillWavesPerEu) void paged_prefill_kernel(PrefillArgs a) {
   prefill_body<W, false, FP8, SH, LT>(a);
+}
+
+// Pipelined long tiles: two waves per SIMD, two workgroups of four waves or
+// one of eight per CU.
+template <int W, int NW, bool FP8>
+__global__ __launch_bounds__(W * 64, 2) void paged_prefill_pipe_kernel(PrefillArgs a) {
+  pipe_body<W, NW, false, FP8>(a);
 }
 
 // Ragged prefill: contiguous K/V rows [nnz_kv, Hkv, 128]; any 16 consecutive
@@ -1168,6 +1879,7 @@ struct loom_paged_prefill_plan {
   loom_paged_prefill_plan_info_t info{};
   uint32_t tile_cols = 16;  // flattened columns per workgroup
   uint32_t long_groups = 1;  // long tiles: wave groups splitting the K/V blocks
+  bool pipe = false;         // long tiles: the pipelined kernel (PipeWave)
   uint32_t tile_layer = 0;   // serpentine tile order layer (PrefillArgs::tile_layer)
   bool tile_interleave = false;  // PrefillArgs::tile_interleave
 };
@@ -1224,9 +1936,6 @@ loom_status_t prefill_grid(uint64_t batch, uint64_t nnz_qo, uint64_t hq, uint64_
 #ifndef LOOM_PREFILL_LONG_MIN_GRID
 #define LOOM_PREFILL_LONG_MIN_GRID 256
 #endif
-#ifndef LOOM_PREFILL_LONG_GROUPS
-#define LOOM_PREFILL_LONG_GROUPS 2
-#endif
 loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
                                 uint64_t nnz_qo, uint64_t hq, uint64_t hkv, bool long_ok,
                                 bool long_default, uint32_t *tile_cols, bool *long_tile,
@@ -1259,6 +1968,40 @@ loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
   }
   *tile_cols = long_requests && grid64 >= LOOM_PREFILL_WIDE_MIN_GRID ? 64 : 16;
   return LOOM_OK;
+}
+
+// The kernel of a paged plan.
+template <bool FP8>
+void launch_paged(const loom_paged_prefill_plan &p, dim3 grid, dim3 block, hipStream_t stream,
+                  const PrefillArgs &a) {
+  if (p.info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && p.pipe) {
+    if (p.tile_cols == 128 && p.long_groups == 2)
+      hipLaunchKernelGGL((paged_prefill_pipe_kernel<8, 4, FP8>), grid, block, 0, stream, a);
+    else if (p.tile_cols == 128)
+      hipLaunchKernelGGL((paged_prefill_pipe_kernel<4, 4, FP8>), grid, block, 0, stream, a);
+    else if (p.long_groups == 4)
+      hipLaunchKernelGGL((paged_prefill_pipe_kernel<8, 2, FP8>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((paged_prefill_pipe_kernel<4, 2, FP8>), grid, block, 0, stream, a);
+  } else if (p.info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE) {
+    if constexpr (!FP8)
+      if (p.tile_cols == 128) {
+        hipLaunchKernelGGL((paged_prefill_kernel<4, false, true, 2>), grid, block, 0, stream, a);
+        return;
+      }
+    if (p.long_groups == 2)
+      hipLaunchKernelGGL((paged_prefill_kernel<8, FP8, true, 1>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((paged_prefill_kernel<4, FP8, true, 1>), grid, block, 0, stream, a);
+  } else if (p.info.algorithm == LOOM_PAGED_PREFILL_WIDE_TILE) {
+    hipLaunchKernelGGL((paged_prefill_kernel<4, FP8, true>), grid, block, 0, stream, a);
+  } else if (p.info.waves == 4) {
+    hipLaunchKernelGGL((paged_prefill_kernel<4, FP8>), grid, block, 0, stream, a);
+  } else if (p.info.waves == 8) {
+    hipLaunchKernelGGL((paged_prefill_kernel<8, FP8>), grid, block, 0, stream, a);
+  } else {
+    hipLaunchKernelGGL((paged_prefill_kernel<16, FP8>), grid, block, 0, stream, a);
+  }
 }
 
 loom_status_t require_aligned(const char *name, uintptr_t ptr, uintptr_t alignment,
@@ -1322,23 +2065,49 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
                       : tile_cols == 64 ? LOOM_PAGED_PREFILL_WIDE_TILE
                                         : LOOM_PAGED_PREFILL_ROW_TILE;
   p->tile_cols = tile_cols;
-  // Long tiles of one query tile per wave (grids too small for two): two
-  // groups of four waves split each tile's K/V blocks, halving the longest
-  // tiles' serial block walk, when the grid fits one round of two such
-  // workgroups per CU or the requests are long enough (1024 rows on average)
-  // that the heaviest tiles dominate.  Measured (GQA4 32/8, BF16 / FP8 pages,
-  // two groups against one): 1 x 512 rows -6% / -15%, 1 x 1024 -2% / -16%,
-  // 1 x 1536 -10% / +2%, and 2 x 512 rows (520 workgroups, a second round)
-  // +6% / -4%.  Long tiles of two query tiles per wave (one such 8-wave
-  // workgroup per CU) split into two groups only on grids of at most two
-  // workgroups per CU: 1 x 2048 rows -11% / -13%, but
-  // 1 x 3072 +16%, 1 x 4096 +27%, 1 x 8192 +25% and 4 x 2048 +36% (the
-  // 8-wave, 2-tile workgroup holds two waves per SIMD and 70 KB of LDS).
-  const bool two_per_cu = grid <= 2 * (uint64_t)provider->dev.cus;
-  const bool grouped = long_tile &&
-                       ((tile_cols == 64 && (two_per_cu || spec->nnz_qo >= 1024 * spec->batch_size)) ||
-                        (tile_cols == 128 && two_per_cu));
-  p->long_groups = grouped ? LOOM_PREFILL_LONG_GROUPS : 1;
+  // The long tiles' kernel and wave groups.  Microseconds on GQA4 32/8, BF16,
+  // one box (plain: LongWave; pipe: PipeWave).
+  //
+  // 128 columns: the pipelined kernel, in two groups of four waves when the
+  // grid holds at most two workgroups per CU.  Its two workgroups per CU walk
+  // long ranges faster, but hide less of a workgroup's start and end than the
+  // plain kernel's three, so batches of requests whose grids run for more
+  // than about two rounds keep the plain kernel on BF16 pages (FP8 pages,
+  // whose plain walk is slower, do not).  plain / pipe: 1 x 2048 rows 53.7 /
+  // 48.5, 1 x 4096 139 / 134, 1 x 8192 513 / 502, 2 x 2048 89 / 76, 8 x 256
+  // 18.9 / 16.5, 8 x 512 40.8 / 38.9, 16 x 256 34.3 / 32.7; 8 x 1024 89.6 /
+  // 93.8, 16 x 512 67.8 / 75.6, 4 x 2048 146.5 / 147.5 (FP8 4 x 2048 157 /
+  // 147); 4 x 512 rows behind 2048-16384 tokens 473 / 384 (FP8 557 / 427).
+  //
+  // 64 columns (grids too small for 128), where the pool may hold contexts
+  // longer than the prompts: the pipelined kernel with two column waves, in
+  // two groups (two workgroups per CU), or in four where the grid holds at
+  // most one workgroup per CU.  plain / two groups / four: 1 x 512 rows 12.9 /
+  // 12.8 / 13.8, 1 x 1024 21.5 / 20.8 / 30.4, 1 x 1536 37.8 / 34.8 / 47.3, 2 x
+  // 512 16.0 / 16.6 / 16.6; 512 rows behind 15872 tokens 276 / 179 / 150.
+  // A pool that holds hardly more than the prompts keeps the plain kernel:
+  // two groups of four waves, halving the longest tiles' serial block walk,
+  // when the grid fits one round of two such workgroups per CU or the
+  // requests are long enough (1024 rows on average) that the heaviest tiles
+  // dominate (two groups against one: 1 x 512 rows -6%, 1 x 1536 -10%, 2 x 512
+  // +6%).
+  const uint64_t cus = provider->dev.cus, hkv_n = spec->num_kv_heads;
+  const bool two_per_cu = grid <= 2 * cus;
+  const bool fp8_pages = spec->kv_dtype == LOOM_KV_DTYPE_FP8_E4M3;
+  const uint64_t page_rows = spec->page_size ? spec->page_size : loom::kPageSize;
+  const bool roomy = spec->max_num_pages >= (2 * spec->nnz_qo + page_rows - 1) / page_rows;
+  if (long_tile && tile_cols == 128) {
+    p->pipe = fp8_pages || spec->batch_size < 3 || grid <= 5 * cus;
+    p->long_groups = two_per_cu ? 2 : 1;
+  } else if (long_tile && roomy) {
+    p->pipe = true;
+    p->long_groups = grid <= cus ? 4 : 2;
+  } else if (long_tile) {
+    p->long_groups = two_per_cu || spec->nnz_qo >= 1024 * spec->batch_size ? 2 : 1;
+  }
+  // waves per workgroup: column waves (pipelined: 32 columns each, else 16 or
+  // 32) times groups
+  const uint32_t long_waves = (p->pipe ? tile_cols / 32 : 4) * p->long_groups;
   // Serpentine tile order when the whole grid is resident at once (long
   // tiles: three 4-wave workgroups per CU; two 8-wave ones of one tile per
   // wave; one of two tiles per wave).  A second round is dispatched as CUs
@@ -1347,8 +2116,7 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
   // 17.2, 1 x 3072 100.5 -> 98.0, 8 x 256 20.1 -> 19.8; on grids of more
   // than one round 1 x 2048 (two tiles, two groups) 58 -> 70, 1 x 4096 141 ->
   // 147, 4 x 2048 153 -> 163.
-  const uint64_t cus = provider->dev.cus, hkv_n = spec->num_kv_heads;
-  const uint64_t resident = p->long_groups == 2 ? (tile_cols == 128 ? 1 : 2) : 3;
+  const uint64_t resident = p->pipe ? (long_waves == 8 ? 1 : 2) : p->long_groups == 2 ? 2 : 3;
   // Requests' tiles interleaved by their distance from the request's end, so
   // that every request's heaviest tiles are dispatched first (the kernel
   // takes up to 64 requests, whose tile counts one wave holds).  Measured (GQA4
@@ -1365,7 +2133,7 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
 
   p->info.waves = waves;
   p->info.row_tiles = tiles;
-  p->info.block_threads = p->info.waves * 64 * p->long_groups;
+  p->info.block_threads = 64 * (long_tile ? long_waves : p->info.waves);
   p->info.grid_blocks = grid;
   p->info.flags = opt.flags;
   *out = p;
@@ -1460,49 +2228,10 @@ loom_status_t loom_paged_prefill_enqueue(const loom_paged_prefill_plan_t *plan,
   a.tile_interleave = plan->tile_interleave ? 1 : 0;
   hipStream_t stream = scope->queue->stream;
   const dim3 grid((unsigned)plan->info.grid_blocks), block(plan->info.block_threads);
-  if (fp8) {
-    switch (plan->info.waves) {
-      case 4:
-        if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->tile_cols == 128 && plan->long_groups == 2)
-          hipLaunchKernelGGL((paged_prefill_kernel<8, true, true, 2>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->tile_cols == 128)
-          hipLaunchKernelGGL((paged_prefill_kernel<4, true, true, 2>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->long_groups == 2)
-          hipLaunchKernelGGL((paged_prefill_kernel<8, true, true, 1>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE)
-          hipLaunchKernelGGL((paged_prefill_kernel<4, true, true, 1>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_WIDE_TILE)
-          hipLaunchKernelGGL((paged_prefill_kernel<4, true, true>), grid, block, 0, stream, a);
-        else
-          hipLaunchKernelGGL((paged_prefill_kernel<4, true>), grid, block, 0, stream, a);
-        break;
-      case 8: hipLaunchKernelGGL((paged_prefill_kernel<8, true>), grid, block, 0, stream, a); break;
-      default:
-        hipLaunchKernelGGL((paged_prefill_kernel<16, true>), grid, block, 0, stream, a);
-        break;
-    }
-  } else {
-    switch (plan->info.waves) {
-      case 4:
-        if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->tile_cols == 128 && plan->long_groups == 2)
-          hipLaunchKernelGGL((paged_prefill_kernel<8, false, true, 2>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->tile_cols == 128)
-          hipLaunchKernelGGL((paged_prefill_kernel<4, false, true, 2>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->long_groups == 2)
-          hipLaunchKernelGGL((paged_prefill_kernel<8, false, true, 1>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE)
-          hipLaunchKernelGGL((paged_prefill_kernel<4, false, true, 1>), grid, block, 0, stream, a);
-        else if (plan->info.algorithm == LOOM_PAGED_PREFILL_WIDE_TILE)
-          hipLaunchKernelGGL((paged_prefill_kernel<4, false, true>), grid, block, 0, stream, a);
-        else
-          hipLaunchKernelGGL((paged_prefill_kernel<4, false>), grid, block, 0, stream, a);
-        break;
-      case 8: hipLaunchKernelGGL((paged_prefill_kernel<8, false>), grid, block, 0, stream, a); break;
-      default:
-        hipLaunchKernelGGL((paged_prefill_kernel<16, false>), grid, block, 0, stream, a);
-        break;
-    }
-  }
+  if (fp8)
+    launch_paged<true>(*plan, grid, block, stream, a);
+  else
+    launch_paged<false>(*plan, grid, block, stream, a);
   return loom::record_launch(scope, hipGetLastError(), err);
 }
 

@@ -1,0 +1,141 @@
+"""GPU parity of the pipelined long-tile prefill kernels (32-token blocks in an
+LDS ring, products and softmax of neighbouring blocks interleaved) at the
+sizes where they can go wrong: remainders of the 64- and 128-column tiles,
+causal ranges of one block and of several 64-block index windows, odd 16-row
+block counts, wave groups with no block of their own, scores that move the
+reference max, and every page form.  Against the oracle where it is quick and
+against the 16-column algorithm on the same pages otherwise, within the
+attention tolerance (gates/paged_batch_decode.rs:18-19: the weights are
+rounded to BF16, at most 2^-9 each, far inside it)."""
+import numpy as np
+import pytest
+
+from gpu_util import PrefillRunner, compare_decode, seeded_normal_bf16
+from test_gpu_prefill import ragged_meta
+from test_gpu_prefill_wide import assert_close, paged_pair
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def L():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    import loom_infer_hip as L
+    return L
+
+
+# (hq, hkv, query rows, kv lengths): pools with room for long contexts, so the
+# 64-column forms run pipelined
+SMALL = [
+    (32, 8, [1], [1]),                       # one token
+    (32, 8, [16], [33]),                     # one tile, a second block of one token
+    (32, 8, [17, 33], [1040, 2065]),         # index windows, odd blocks
+    (28, 4, [19, 5], [300, 77]),             # a group of 7 across tiles
+    (8, 8, [64, 65, 63], [64, 65, 1500]),    # group 1: tiles of 64 rows, whole prompts
+    (8, 1, [9, 3, 40], [31, 32, 1056]),      # MQA
+]
+
+
+@pytest.mark.parametrize("shape", SMALL, ids=lambda s: f"{s[0]}x{s[1]}_{sum(s[2])}of{sum(s[3])}")
+def test_small_grids_match_the_oracle(L, oracle, shape):
+    hq, hkv, qo_lens, kv_lens = shape
+    rng = np.random.default_rng(sum(kv_lens) + 77)
+    pool = 2 * sum((n + 15) // 16 for n in kv_lens) + 2 * sum(qo_lens)
+    qo, ip, ix, last = ragged_meta(rng, qo_lens, kv_lens, pool)
+    B, nnz = len(qo_lens), int(qo[-1])
+    q = seeded_normal_bf16(oracle, rng, nnz * hq * 128)
+    k = seeded_normal_bf16(oracle, rng, pool * 16 * hkv * 128)
+    v = seeded_normal_bf16(oracle, rng, pool * 16 * hkv * 128)
+    ref = oracle.prefill(oracle.prefill_spec(B, nnz, pool, hq, hkv), q, k, v, qo, ip, ix, last)
+    r = PrefillRunner(L, B, nnz, pool, hq, hkv, tile_cols="long")
+    out, lse = r.run(q, k, v, qo, ip, ix, last)
+    compare_decode(oracle, out, lse, *ref)
+
+
+# (hq, hkv, rows, kv lengths, threads): the forms a plan takes by itself
+PLANS = [
+    (32, 8, [512], [1500], 512),                    # 64 columns, four groups
+    (32, 8, [500, 90], [700, 2300], 256),           # 64 columns, two groups
+    (32, 8, [2048], [2177], 512),                   # 128 columns, two groups
+    (32, 8, [900, 1100, 1000], [900, 1100, 1900], 256),  # 128 columns, one group
+]
+
+
+@pytest.mark.parametrize("form", ["bf16", "bf16_hnd", "bf16_page64", "fp8", "fp8_hnd_page32"])
+@pytest.mark.parametrize("plan", PLANS, ids=lambda s: f"{s[4]}t_{sum(s[2])}of{sum(s[3])}")
+def test_planned_forms_match_row_tiles(L, oracle, plan, form):
+    import torch
+    hq, hkv, qo_lens, kv_lens, threads = plan
+    P = 64 if "64" in form else 32 if "32" in form else 16
+    rng = np.random.default_rng(sum(kv_lens) + P)
+    pages = [(n + P - 1) // P for n in kv_lens]
+    nnz, B = sum(qo_lens), len(qo_lens)
+    pool = max(sum(pages) + 3, (2 * nnz + P - 1) // P)
+    ip = np.concatenate([[0], np.cumsum(pages)]).astype(np.int32)
+    ix = rng.permutation(pool)[: ip[-1]].astype(np.int32)
+    last = np.array([n - (p - 1) * P for n, p in zip(kv_lens, pages)], np.int32)
+    qo = np.concatenate([[0], np.cumsum(qo_lens)]).astype(np.int32)
+    g = torch.Generator(device="cuda").manual_seed(nnz)
+    q = torch.randn(nnz * hq * 128, device="cuda", generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(pool * P * hkv * 128, device="cuda", generator=g) for _ in range(2))
+    kw, scales = {"kv_page_size": P}, None
+    if "hnd" in form:
+        kw["kv_layout"] = "HND"
+    if form.startswith("fp8"):
+        kw["kv_dtype"], scales = "fp8_e4m3", [0.8, 1.3]
+        k, v = (x.to(torch.float8_e4m3fn).view(torch.uint8) for x in (k, v))
+    else:
+        k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    p = L.PrefillProvider.load(0).plan_bf16_paged(
+        L.Bf16PagedPrefillSpec(B, nnz, pool, hq, hkv, **kw))
+    assert p.algorithm == "long_tile" and p.info.block_threads == threads
+    res = paged_pair(L, B, nnz, pool, hq, hkv, q, k, v, qo, ip, ix, last, spec_kw=kw,
+                     scales=scales, tile="long")
+    assert not np.any(np.isnan(oracle.bf16_to_f32(res[0][0])))
+    assert_close(oracle, res)
+
+
+def test_growing_scores_move_the_reference_max(L, oracle):
+    """Keys that grow along the context: the normalizer passes its refresh
+    threshold again and again (scores rise by thousands in the log2 domain),
+    early tokens' weights vanish, and the result stays the oracle's.  A score's
+    FP32 rounding is up to 2^-24 of its magnitude (2^-9 here), so the LSE and
+    the weights keep within the gate."""
+    rng = np.random.default_rng(5)
+    hq, hkv, rows, n = 16, 4, 40, 900
+    pool = 200
+    qo, ip, ix, last = ragged_meta(rng, [rows], [n], pool)
+    q = np.abs(rng.standard_normal((rows, hq, 128), dtype=np.float32))
+    k = rng.standard_normal((pool, 16, hkv, 128), dtype=np.float32)
+    at = {int(p): i for i, p in enumerate(ix)}
+    for p, i in at.items():
+        for t in range(16):
+            k[p, t] = np.abs(k[p, t]) * (16 * i + t) / 24.0
+    qb, kb = oracle.bf16_from_f32(q.ravel()), oracle.bf16_from_f32(k.ravel())
+    v = seeded_normal_bf16(oracle, rng, pool * 16 * hkv * 128)
+    ref = oracle.prefill(oracle.prefill_spec(1, rows, pool, hq, hkv), qb, kb, v, qo, ip, ix, last)
+    r = PrefillRunner(L, 1, rows, pool, hq, hkv, tile_cols="long")
+    out, lse = r.run(qb, kb, v, qo, ip, ix, last)
+    assert float(np.nanmax(np.abs(ref[1]))) > 500
+    compare_decode(oracle, out, lse, *ref)
+
+
+@pytest.mark.parametrize("batch", [65, 130])
+def test_more_requests_than_a_wave(L, oracle, batch):
+    """Batches past 64 requests take the workgroup-wide search for a tile."""
+    rng = np.random.default_rng(batch)
+    hq, hkv = 8, 2
+    kv_lens = [int(x) for x in rng.integers(1, 70, size=batch)]
+    qo_lens = [int(rng.integers(1, n + 1)) for n in kv_lens]
+    pool = sum((n + 15) // 16 for n in kv_lens) + 2 * sum(qo_lens) // 16 + 3
+    qo, ip, ix, last = ragged_meta(rng, qo_lens, kv_lens, pool)
+    nnz = int(qo[-1])
+    q = seeded_normal_bf16(oracle, rng, nnz * hq * 128)
+    k = seeded_normal_bf16(oracle, rng, pool * 16 * hkv * 128)
+    v = seeded_normal_bf16(oracle, rng, pool * 16 * hkv * 128)
+    ref = oracle.prefill(oracle.prefill_spec(batch, nnz, pool, hq, hkv), q, k, v, qo, ip, ix, last)
+    for tile in ("long", 16):
+        r = PrefillRunner(L, batch, nnz, pool, hq, hkv, tile_cols=tile)
+        out, lse = r.run(q, k, v, qo, ip, ix, last)
+        compare_decode(oracle, out, lse, *ref)
