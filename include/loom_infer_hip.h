@@ -815,8 +815,9 @@ typedef struct loom_ragged_prefill_plan loom_ragged_prefill_plan_t;
 
 typedef struct loom_ragged_prefill_plan_info {
   loom_ragged_prefill_spec_t spec;
-  int32_t algorithm;          /* LOOM_PAGED_PREFILL_ROW_TILE or _WIDE_TILE: the same
-                                 kernel designs */
+  int32_t algorithm;          /* LOOM_PAGED_PREFILL_ROW_TILE, _WIDE_TILE or _LONG_TILE: the
+                                 same kernel designs (LONG_TILE with the weights as a BF16
+                                 high part and residual; chosen by the plan only) */
   uint32_t waves;
   uint64_t row_tiles;
   uint32_t block_threads;

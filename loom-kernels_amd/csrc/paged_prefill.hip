@@ -1868,6 +1868,11 @@ __global__ __launch_bounds__(W * 64, kPrefillWavesPerEu) void ragged_prefill_ker
   prefill_body<W, true, false, SH>(a);
 }
 
+template <int W, int NW>
+__global__ __launch_bounds__(W * 64, 2) void ragged_prefill_pipe_kernel(PrefillArgs a) {
+  pipe_body<W, NW, true, false>(a);
+}
+
 }  // namespace
 
 // ---- provider / plan / enqueue -----------------------------------------------
@@ -1886,6 +1891,10 @@ struct loom_paged_prefill_plan {
 
 struct loom_ragged_prefill_plan {
   loom_ragged_prefill_plan_info_t info{};
+  uint32_t tile_cols = 16;   // flattened columns per workgroup
+  uint32_t long_groups = 1;  // long tiles: wave groups splitting the K/V blocks
+  uint32_t tile_layer = 0;   // PrefillArgs::tile_layer
+  bool tile_interleave = false;  // PrefillArgs::tile_interleave
 };
 
 namespace {
@@ -1960,7 +1969,7 @@ loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
   // Long prompts on BF16 pages take the long tiles, from a smaller grid than
   // the wide tiles need (see the algorithm's measurements in the plan's
   // documentation).
-  *long_tile = long_requests && long_ok && long_default && LOOM_PREFILL_LONG_DEFAULT &&
+  *long_tile = long_requests && long_default && LOOM_PREFILL_LONG_DEFAULT &&
                grid64 >= LOOM_PREFILL_LONG_MIN_GRID;
   if (*long_tile) {
     *tile_cols = (cols / 128) * hkv >= kLongTwoMinGrid ? 128 : 64;
@@ -2084,7 +2093,9 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
   // two groups (two workgroups per CU), or in four where the grid holds at
   // most one workgroup per CU.  plain / two groups / four: 1 x 512 rows 12.9 /
   // 12.8 / 13.8, 1 x 1024 21.5 / 20.8 / 30.4, 1 x 1536 37.8 / 34.8 / 47.3, 2 x
-  // 512 16.0 / 16.6 / 16.6; 512 rows behind 15872 tokens 276 / 179 / 150.
+  // 512 16.0 / 16.6 / 16.6; 512 rows behind 15872 tokens 276 / 179 / 150.  On
+  // grids of a second round its starts and ends show unless the requests are
+  // long (12 x 100 rows 11.1 / 20.2, 6 x 200 12.1 / 21.0): the plain kernel.
   // A pool that holds hardly more than the prompts keeps the plain kernel:
   // two groups of four waves, halving the longest tiles' serial block walk,
   // when the grid fits one round of two such workgroups per CU or the
@@ -2099,7 +2110,7 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
   if (long_tile && tile_cols == 128) {
     p->pipe = fp8_pages || spec->batch_size < 3 || grid <= 5 * cus;
     p->long_groups = two_per_cu ? 2 : 1;
-  } else if (long_tile && roomy) {
+  } else if (long_tile && roomy && (two_per_cu || spec->nnz_qo >= 1024 * spec->batch_size)) {
     p->pipe = true;
     p->long_groups = grid <= cus ? 4 : 2;
   } else if (long_tile) {
@@ -2251,19 +2262,46 @@ loom_status_t loom_prefill_provider_plan_bf16_ragged(
   uint32_t tile_cols = 16;
   bool long_tile = false;
   loom_status_t rc = prefill_tile_cols(opt.flags, waves, spec->batch_size, spec->nnz_qo,
-                                       spec->num_query_heads, spec->num_kv_heads, false, false,
+                                       spec->num_query_heads, spec->num_kv_heads, false, true,
                                        &tile_cols, &long_tile, err);
   if (rc) return rc;
   uint64_t tiles = 0, grid = 0;
   rc = prefill_grid(spec->batch_size, spec->nnz_qo, spec->num_query_heads, spec->num_kv_heads,
                     tile_cols, &tiles, &grid, err);
   if (rc) return rc;
+  // Long tiles, always pipelined (weights as high part and residual), where
+  // the wide tiles ran before and from grids half as large.  Microseconds,
+  // GQA4 32/8, before / now: 1 x 512 rows 19.8 / 15.0, 1 x 1024 43.3 / 22.9, 1 x
+  // 2048 88 / 58, 1 x 8192 1102 / 644, 4 x 2048 329 / 213, 8 x 256 27.1 / 17.9, 4
+  // x 512 rows behind 7680 592 / 323.  Short requests on 64-column grids of
+  // more than one round (two workgroups per CU) keep the row and wide tiles:
+  // 12 x 100 rows 12.1 / 20.3, 6 x 200 17.2 / 21.1 (but 6 x 150, one round,
+  // 18.6 / 12.7, and 1 x 1536 63.8 / 40.7).
+  const uint64_t cus = provider->dev.cus, hkv_n = spec->num_kv_heads, b = spec->batch_size;
+  if (long_tile && tile_cols == 64 && grid > 2 * cus && spec->nnz_kv < 512 * b) {
+    long_tile = false;
+    const uint64_t cols = spec->nnz_qo * (spec->num_query_heads / hkv_n);
+    tile_cols = (cols / 64) * hkv_n >= LOOM_PREFILL_WIDE_MIN_GRID ? 64 : 16;
+    rc = prefill_grid(b, spec->nnz_qo, spec->num_query_heads, hkv_n, tile_cols, &tiles, &grid, err);
+    if (rc) return rc;
+  }
   auto *p = new loom_ragged_prefill_plan;
   p->info.spec = *spec;
-  p->info.algorithm = tile_cols == 64 ? LOOM_PAGED_PREFILL_WIDE_TILE : LOOM_PAGED_PREFILL_ROW_TILE;
+  p->info.algorithm = long_tile         ? LOOM_PAGED_PREFILL_LONG_TILE
+                      : tile_cols == 64 ? LOOM_PAGED_PREFILL_WIDE_TILE
+                                        : LOOM_PAGED_PREFILL_ROW_TILE;
+  p->tile_cols = tile_cols;
+  // Wave groups, serpentine order and interleaving as for the paged plan.
+  if (long_tile) {
+    p->long_groups = tile_cols == 128 ? (grid <= 2 * cus ? 2 : 1) : (grid <= cus ? 4 : 2);
+    const uint32_t long_waves = tile_cols / 32 * p->long_groups;
+    const uint64_t resident = long_waves == 8 ? 1 : 2;
+    p->tile_interleave = b <= 16 && (b >= 3 || (b == 2 && grid > 2 * cus * resident));
+    p->tile_layer = hkv_n > 0 && cus >= hkv_n && grid <= cus * resident ? (uint32_t)(cus / hkv_n) : 0;
+  }
   p->info.waves = waves;
   p->info.row_tiles = tiles;
-  p->info.block_threads = p->info.waves * 64;
+  p->info.block_threads = 64 * (long_tile ? tile_cols / 32 * p->long_groups : p->info.waves);
   p->info.grid_blocks = grid;
   p->info.workspace_numel = 0;
   *out = p;
@@ -2330,9 +2368,20 @@ loom_status_t loom_ragged_prefill_enqueue(const loom_ragged_prefill_plan_t *plan
   a.blocks_lg = 0;
   hipStream_t stream = scope->queue->stream;
   const dim3 grid((unsigned)plan->info.grid_blocks), block(plan->info.block_threads);
+  a.tile_layer = (int32_t)plan->tile_layer;
+  a.tile_interleave = plan->tile_interleave ? 1 : 0;
   switch (plan->info.waves) {
     case 4:
-      if (plan->info.algorithm == LOOM_PAGED_PREFILL_WIDE_TILE)
+      if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->tile_cols == 128 &&
+          plan->long_groups == 2)
+        hipLaunchKernelGGL((ragged_prefill_pipe_kernel<8, 4>), grid, block, 0, stream, a);
+      else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->tile_cols == 128)
+        hipLaunchKernelGGL((ragged_prefill_pipe_kernel<4, 4>), grid, block, 0, stream, a);
+      else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->long_groups == 4)
+        hipLaunchKernelGGL((ragged_prefill_pipe_kernel<8, 2>), grid, block, 0, stream, a);
+      else if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE)
+        hipLaunchKernelGGL((ragged_prefill_pipe_kernel<4, 2>), grid, block, 0, stream, a);
+      else if (plan->info.algorithm == LOOM_PAGED_PREFILL_WIDE_TILE)
         hipLaunchKernelGGL((ragged_prefill_kernel<4, true>), grid, block, 0, stream, a);
       else
         hipLaunchKernelGGL(ragged_prefill_kernel<4>, grid, block, 0, stream, a);

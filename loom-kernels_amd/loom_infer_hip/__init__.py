@@ -1079,7 +1079,7 @@ class Bf16RaggedPrefillPlan:
 
     @property
     def algorithm(self) -> str:
-        return {1: "row_tile", 2: "wide_tile"}[self.info.algorithm]
+        return {1: "row_tile", 2: "wide_tile", 3: "long_tile"}[self.info.algorithm]
 
     @property
     def workspace_required_numel(self) -> int:

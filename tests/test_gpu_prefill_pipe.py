@@ -139,3 +139,41 @@ def test_more_requests_than_a_wave(L, oracle, batch):
         r = PrefillRunner(L, batch, nnz, pool, hq, hkv, tile_cols=tile)
         out, lse = r.run(q, k, v, qo, ip, ix, last)
         compare_decode(oracle, out, lse, *ref)
+
+
+# (hq, hkv, rows, kv lengths): ragged plans that run the pipelined tiles (64
+# columns in four and two groups, 128 columns in two and one)
+RAGGED = [
+    (32, 8, [515], [515]),
+    (32, 8, [300, 257], [1031, 300]),
+    (32, 8, [2048], [2090]),
+    (16, 2, [700, 513, 400], [700, 1300, 433]),
+    (28, 4, [401, 999], [401, 1033]),
+]
+
+
+@pytest.mark.parametrize("shape", RAGGED, ids=lambda s: f"{s[0]}x{s[1]}_{sum(s[2])}of{sum(s[3])}")
+def test_ragged_plans_match_row_tiles(L, oracle, shape):
+    """The ragged contract's pipelined tiles keep 16 bits of every weight and
+    FP32 normalizers, as its 16-column algorithm does: outputs differ by BF16
+    rounding flips at most (one ulp of values below 4: 2^-6) and the LSE by
+    FP32 summation order."""
+    from gpu_util import RaggedRunner, bf16_host, to_dev_i32
+    import torch
+    hq, hkv, qo_lens, kv_lens = shape
+    qo = np.concatenate([[0], np.cumsum(qo_lens)]).astype(np.int32)
+    kv = np.concatenate([[0], np.cumsum(kv_lens)]).astype(np.int32)
+    B, nq, nkv = len(qo_lens), int(qo[-1]), int(kv[-1])
+    g = torch.Generator(device="cuda").manual_seed(nq)
+    q, k, v = (torch.randn(n * h * 128, device="cuda", generator=g).to(torch.bfloat16)
+               for n, h in ((nq, hq), (nkv, hkv), (nkv, hkv)))
+    res = []
+    for tile in (0, 16):
+        r = RaggedRunner(L, B, nq, nkv, hq, hkv, tile_cols=tile)
+        assert r.plan.algorithm == ("row_tile" if tile else "long_tile")
+        out, lse = r.run_dev(q, k, v, to_dev_i32(qo), to_dev_i32(kv))
+        res.append((oracle.bf16_to_f32(bf16_host(out)), lse.cpu().numpy()))
+    (o, l), (eo, el) = res
+    assert np.all(np.isfinite(o)) and np.abs(o - eo).max() <= 2.0 ** -6
+    assert np.mean(o != eo) < 0.02
+    assert np.abs(l - el).max() <= 1e-5
