@@ -1292,6 +1292,7 @@ struct loom_paged_decode_plan {
 };
 
 struct loom_single_decode_plan {
+  uint32_t partitions = 1;  // token partitions of the two-kernel form (1: one kernel)
   loom_single_decode_spec_t spec;
   uint32_t group_tile = 1, group_tiles = 1;
 };
@@ -1783,6 +1784,23 @@ loom_status_t loom_paged_decode_enqueue_bf16_no_alloc(
 
 
 // ---- contiguous single decode: plans and enqueue -------------------------------
+// Token partitions of a direct plan.  One workgroup per (kv-head, tile) walks
+// its tokens 16 at a time over four waves on a handful of CUs, 0.56 us per 64
+// tokens; from 640 tokens on the split-K kernels (one wave per partition, then
+// a merge) are faster although they are two launches.  Partitions of at least
+// two 16-token blocks, up to 64 (one round trip of the merge), of eight blocks
+// on long contexts, and at most 1024 waves.  Microseconds, one kernel / two
+// (Hq x Hkv): 512 tokens 7.7 / 8.0 (32x8), 7.3 / 8.0 (32x32); 1024 12.2 / 8.2,
+// 11.7 / 8.1; 4096 39.0 / 10.0, 42.3 / 15.6, 38.8 / 10.2 (32x4); 16384 157 /
+// 16.1, 171 / 43.5, 145 / 13.5 (8x1).
+constexpr uint64_t kSingleSplitMin = 640;
+static uint32_t single_partitions(uint64_t kv_len, uint64_t members) {
+  if (kv_len < kSingleSplitMin) return 1;
+  const uint64_t blocks = (kv_len + 15) / 16;
+  const uint64_t parts = blocks <= 512 ? std::min<uint64_t>(64, blocks / 2) : blocks / 8;
+  return (uint32_t)std::max<uint64_t>(1, std::min(parts, 1024 / members));
+}
+
 loom_status_t loom_decode_provider_plan_bf16(const loom_decode_provider_t *provider,
                                              const loom_single_decode_spec_t *spec,
                                              loom_single_decode_plan_t **out, loom_error_t *err) {
@@ -1796,6 +1814,7 @@ loom_status_t loom_decode_provider_plan_bf16(const loom_decode_provider_t *provi
   const uint64_t group = spec->num_query_heads / spec->num_kv_heads;
   p->group_tile = group_tile_for(group);
   p->group_tiles = (uint32_t)((group + p->group_tile - 1) / p->group_tile);
+  p->partitions = single_partitions(spec->kv_len, spec->num_kv_heads * p->group_tiles);
   *out = p;
   return loom::ok(err);
 }
@@ -1833,6 +1852,24 @@ uint64_t loom_single_decode_split_k_workspace_bytes(const loom_single_decode_spl
 }
 
 namespace {
+// The split-K partial kernel and its merge.
+hipError_t launch_split_k(uint32_t group_tile, const DecodeArgs &a, int64_t L, int P, float *ws,
+                          hipStream_t stream) {
+  const uint64_t waves = (uint64_t)P * a.members;
+  const dim3 g3((unsigned)((waves + kWaves - 1) / kWaves)), b3(kThreads);
+  switch (group_tile) {
+    case 1: hipLaunchKernelGGL(single_decode_split_k_kernel<1>, g3, b3, 0, stream, a, L, P, ws); break;
+    case 2: hipLaunchKernelGGL(single_decode_split_k_kernel<2>, g3, b3, 0, stream, a, L, P, ws); break;
+    case 4: hipLaunchKernelGGL(single_decode_split_k_kernel<4>, g3, b3, 0, stream, a, L, P, ws); break;
+    default: hipLaunchKernelGGL(single_decode_split_k_kernel<8>, g3, b3, 0, stream, a, L, P, ws); break;
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(single_decode_split_k_merge_kernel, dim3((unsigned)a.hq), dim3(kMergeWaves * 64),
+                     0, stream, a, P, (const float *)ws);
+  return hipGetLastError();
+}
+
 // decode.rs:1683-1696 checks 4-byte alignment for its packed pairs, and so
 // do these: their 16-byte accesses need no more on gfx950 (global and buffer
 // accesses run in unaligned mode).
@@ -1870,9 +1907,21 @@ loom_status_t loom_single_decode_enqueue(const loom_single_decode_plan_t *plan,
   if ((rc = require_aligned("O", l[3]->ptr, 4, err))) return rc;
   DecodeArgs a = single_args(s, plan->group_tiles, l[0]->ptr, l[1]->ptr, l[2]->ptr, l[3]->ptr,
                              l[4]->ptr);
-  const dim3 g3((unsigned)(s.num_kv_heads * plan->group_tiles)), b3(kThreads);
   hipStream_t stream = scope->queue->stream;
   const int64_t L = (int64_t)s.kv_len;
+  if (plan->partitions > 1) {
+    // The partial states live in the queue's scratch.  Where it is missing and
+    // cannot be allocated (a captured stream without a reservation, no
+    // memory) the one-kernel form runs.
+    uint8_t *ws = nullptr;
+    const uint64_t bytes = s.num_query_heads * plan->partitions * loom::kStateWidth * 4;
+    if (loom::queue_workspace(scope->queue, bytes, false, &ws, nullptr) == LOOM_OK)
+      return loom::record_launch(
+          scope, launch_split_k(plan->group_tile, a, L, (int)plan->partitions, (float *)ws, stream),
+          err);
+    (void)hipGetLastError();
+  }
+  const dim3 g3((unsigned)(s.num_kv_heads * plan->group_tiles)), b3(kThreads);
   switch (plan->group_tile) {
     case 1: hipLaunchKernelGGL(single_decode_kernel<1>, g3, b3, 0, stream, a, L); break;
     case 2: hipLaunchKernelGGL(single_decode_kernel<2>, g3, b3, 0, stream, a, L); break;

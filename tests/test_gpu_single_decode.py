@@ -154,3 +154,39 @@ def test_split_k_rejections_submit_nothing(L):
     comp = scope.finish()
     assert comp.submitted() == 0
     comp.wait()
+
+
+@pytest.mark.parametrize("kv_len,hq,hkv", [(639, 32, 8), (640, 32, 8), (641, 8, 1),
+                                           (1023, 28, 4), (2049, 32, 32), (8193, 32, 4)])
+def test_direct_plan_around_its_partitions(L, oracle, kv_len, hq, hkv):
+    """Direct plans of 640 tokens or more run as partitions and a merge in the
+    queue's scratch; a captured stream without a reservation keeps the one
+    kernel, and with one replays the two.  All within the attention gate of
+    the oracle; the two captures differ from the eager result by FP32 summation
+    order at most (one BF16 ulp, 2^-8 of values below 1)."""
+    import torch
+    q, k, v = fixture(oracle, kv_len, hq, hkv, 0x5100 + kv_len)
+    spec = L.Bf16SingleDecodeSpec(kv_len, hq, hkv)
+    ref = oracle.single_decode(oracle.single_spec(kv_len, hq, hkv), q, k, v)
+    out, lse = run_single(L, spec, q, k, v)
+    compare_decode(oracle, out, lse, *ref)
+    plan = L.DecodeProvider.load(0).plan_bf16(spec)
+    tq, tk, tv = to_dev_bf16(q), to_dev_bf16(k), to_dev_bf16(v)
+    for reserve in (0, 1 << 24):
+        o = torch.full((spec.output_numel,), float("nan"), dtype=torch.bfloat16, device="cuda")
+        le = torch.full((spec.lse_numel,), float("nan"), dtype=torch.float32, device="cuda")
+        gq = L.GraphQueue(0, 1)
+        if reserve:
+            gq.reserve_workspace(reserve)
+        torch.cuda.synchronize()
+        b = gq.bindings(5)
+        args = L.Bf16SingleDecodeArgs(b.bind_read(tq), b.bind_read(tk), b.bind_read(tv),
+                                      b.bind_read_write(o).write(), b.bind_read_write(le).write())
+        graph = gq.capture(b, lambda scope: plan.enqueue_into(scope, args)).instantiate()
+        for _ in range(3):
+            o.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.launch().wait()
+            compare_decode(oracle, bf16_host(o), le.cpu().numpy(), *ref)
+            if reserve:
+                assert np.array_equal(bf16_host(o), out)
