@@ -91,12 +91,30 @@ struct PrefillArgs {
   // FP8 E4M3 pages: device [k_scale, v_scale] (K = fp8 * k_scale, V = fp8 *
   // v_scale); null for BF16 pages.
   const float *kv_scales;
+  // Split row tiles: workgroups per (tile, kv-head), each over an equal share
+  // of the tile's blocks, and their column states: state c of tile rank m,
+  // kv-head h and split s at ((s * row_tiles + m) * Hkv + h) * 16 + c, as
+  // (max_log2, normalizer, 2 pad, acc[128]).
+  int32_t splits;
+  int32_t row_tiles;
+  float *states;
 };
+
+// Floats of a split state.
+constexpr int kSplitState = 132;
+constexpr int kMaxSplits = 16;
+// Splits that a tile of `blocks` 16-row blocks uses of the command's `splits`:
+// at least eight blocks (two per wave) each.
+__host__ __device__ constexpr int tile_splits(int blocks, int splits) {
+  const int most = (blocks + 7) / 8;
+  return splits < most ? splits : most < 1 ? 1 : most;
+}
 
 // ---- locating a workgroup's tile ------------------------------------------------
 // The tile of workgroup blockIdx.x and the request that owns it (wave-uniform).
 struct TileLoc {
   int kvh;
+  int rank;               // place among the grid's tiles
   int tile0;              // tile within the request's columns
   int32_t qs, qe;         // the request's qo_indptr pair
   int32_t ps, pe;         // its page (ragged: kv) indptr pair
@@ -145,11 +163,13 @@ struct LocateSmem {
 // the way (16 requests of 256 BF16 rows, GQA4 32/8: 35.0 -> 34.3 us; 1 x 1024
 // 22.3 -> 21.5, 1 x 512 13.8 -> 12.9; a batch of two on row tiles 14.2 -> 13.5).
 template <int W, bool RAGGED, int TC, bool INTERLEAVE>
-__device__ __forceinline__ bool locate_tile(const PrefillArgs &a, LocateSmem<W> &sm, TileLoc &t) {
+__device__ __forceinline__ bool locate_tile(const PrefillArgs &a, LocateSmem<W> &sm, TileLoc &t,
+                                            int split = 0) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   t.kvh = (int)(blockIdx.x % a.hkv);
-  const int64_t n_tiles = (int64_t)(gridDim.x / a.hkv), m = blockIdx.x / a.hkv;
+  const int64_t n_tiles = a.row_tiles, m = (int64_t)(blockIdx.x / a.hkv) - split * n_tiles;
+  t.rank = (int)m;
   int64_t rank = m;
   if (a.tile_layer > 0) {
     // Serpentine: every other layer of tile_layer workgroups (one per CU of
@@ -364,7 +384,11 @@ struct PrefillPage {
   u32x4 v[4];
 };
 
-// elem0: element offset of the block's first row for kv-head 0.
+// elem0: element offset of the block's first row for kv-head 0.  KROWS: K as
+// whole rows, in V's layout (staged through LDS before use): four rows per
+// load instruction take 18 cycles of the CU's load path, the fragment
+// layout's 16 rows 64.
+template <bool KROWS>
 __device__ __forceinline__ void load_prefill_page(PrefillPage &p, const PrefillArgs &a,
                                                   int64_t elem0, int rows, int lane, int kvh) {
   const int col = lane & 15, quad = lane >> 4;
@@ -373,7 +397,9 @@ __device__ __forceinline__ void load_prefill_page(PrefillPage &p, const PrefillA
   const __amdgpu_buffer_rsrc_t rv = page_rows_rsrc(a.v + first, rows, a.row_elems);
   const int row_bytes = a.row_elems * 2;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) p.k[c] = load16_rows<false>(rk, col * row_bytes + (32 * c + 8 * quad) * 2);
+  for (int c = 0; c < 4; ++c)
+    p.k[c] = load16_rows<false>(rk, KROWS ? (quad * 4 + c) * row_bytes + col * 16
+                                          : col * row_bytes + (32 * c + 8 * quad) * 2);
 #pragma unroll
   for (int j = 0; j < 4; ++j) p.v[j] = load16_rows<false>(rv, (quad * 4 + j) * row_bytes + col * 16);
 }
@@ -385,6 +411,7 @@ struct PrefillPage8 {
   u32x2 v[4];
 };
 
+template <bool KROWS>
 __device__ __forceinline__ void load_prefill_page(PrefillPage8 &p, const PrefillArgs &a,
                                                   int64_t elem0, int rows, int lane, int kvh) {
   const int col = lane & 15, quad = lane >> 4;
@@ -397,7 +424,9 @@ __device__ __forceinline__ void load_prefill_page(PrefillPage8 &p, const Prefill
   const __amdgpu_buffer_rsrc_t rv =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(v8), 0, bytes, 0x00020000);
 #pragma unroll
-  for (int c = 0; c < 4; ++c) p.k[c] = load8_rows<false>(rk, col * a.row_elems + 32 * c + 8 * quad);
+  for (int c = 0; c < 4; ++c)
+    p.k[c] = load8_rows<false>(rk, KROWS ? (quad * 4 + c) * a.row_elems + col * 8
+                                         : col * a.row_elems + 32 * c + 8 * quad);
 #pragma unroll
   for (int j = 0; j < 4; ++j) p.v[j] = load8_rows<false>(rv, (quad * 4 + j) * a.row_elems + col * 8);
 }
@@ -416,9 +445,14 @@ __device__ __forceinline__ PrefillPage expand(const PrefillPage8 &p) {
 template <bool FP8>
 using PrefillBuf = typename std::conditional<FP8, PrefillPage8, PrefillPage>::type;
 
+// KROWS: pages come with K as whole rows and pass through the wave's LDS tile
+// `kt` (16 rows of kKRowBytes, padded against bank conflicts).
+constexpr int kKRowBytes = 256 + 16;
+template <bool KROWS>
 struct PrefillWave {
   const PrefillArgs &a;
   const u32x4 (*qfrag)[64];
+  uint8_t *kt;
   int lane, col, quad, kvh;
   int64_t end_col;  // causal end (exclusive) of this lane's column, 0 if unused
   float m_run, l_run;
@@ -433,11 +467,22 @@ struct PrefillWave {
 
   // `lt0`: logical token index of the page's first row in the request.
   __device__ void process(const PrefillPage &pg, int64_t lt0) {
+    u32x4 kf[4];
+    if constexpr (KROWS) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<u32x4 *>(kt + (quad * 4 + j) * kKRowBytes + col * 16) = pg.k[j];
+      wave_lds_fence();
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      kf[c] = KROWS ? *reinterpret_cast<const u32x4 *>(kt + col * kKRowBytes + (c * 4 + quad) * 16)
+                    : pg.k[c];
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(pg.k[c]), as_bf16x8(qfrag[c][lane]),
-                                                  s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[c]), as_bf16x8(qfrag[c][lane]), s,
+                                                  0, 0, 0);
     // s[i] = S[token 4 quad + i][column col]; tokens at or past the column's
     // causal end (which also covers the rows past kv_len) are masked.
     const int vis = (int)max<int64_t>(-1, min<int64_t>(16, end_col - lt0));
@@ -490,7 +535,7 @@ struct PrefillWave {
   template <int D, bool FP8, class PageTok, class RowsOf>
   __device__ void prime(PrefillBuf<FP8> (&buf)[D], PageTok page_tok, RowsOf rows_of) {
 #pragma unroll
-    for (int j = 0; j < D - 1; ++j) load_prefill_page(buf[j], a, page_tok(j), rows_of(j), lane, kvh);
+    for (int j = 0; j < D - 1; ++j) load_prefill_page<KROWS>(buf[j], a, page_tok(j), rows_of(j), lane, kvh);
   }
 
   // `primed`: the loads of pages 0..D-2 are already in flight in `buf`.
@@ -502,7 +547,7 @@ struct PrefillWave {
     while (true) {
 #pragma unroll
       for (int s = 0; s < D; ++s) {
-        load_prefill_page(buf[(s + D - 1) % D], a, page_tok(i + D - 1), rows_of(i + D - 1), lane,
+        load_prefill_page<KROWS>(buf[(s + D - 1) % D], a, page_tok(i + D - 1), rows_of(i + D - 1), lane,
                           kvh);
         process(expand(buf[s]), lt_of(i));
         if (++i >= n) return;
@@ -1205,8 +1250,11 @@ constexpr int kLongTwoMinGrid = 512;
 // one 16-column tile per wave, every wave over the whole page range.
 // LT: the long-tile algorithm (SH's columns and block walk; 32-token blocks,
 // query fragments in registers, BF16 P, Vᵀ staged transposed).
-template <int W, bool RAGGED, bool FP8, bool SH, int LT = 0>
+// SPLIT (row tiles): K comes as whole rows, and a.splits workgroups (one: no
+// merge) share the tile's blocks.
+template <int W, bool RAGGED, bool FP8, bool SH, int LT = 0, bool SPLIT = false>
 __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
+  static_assert(!SPLIT || (!SH && !LT), "row tiles");
   static_assert(!SH || W == 4 || (LT >= 1 && W == 8),
                 "wide tiles: four waves; long tiles: four, or two groups of four with one tile");
   static_assert(!LT || SH, "long tiles: the wide tiles' columns");
@@ -1241,7 +1289,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     if (lane + 64 < a.n_indices) tbl1 = a.indices[lane + 64];
   }
   TileLoc loc;
-  if (!locate_tile<W, RAGGED, TC, LT != 0>(a, sm.loc, loc)) return;
+  const int split = SPLIT ? (int)(blockIdx.x / a.hkv) / a.row_tiles : 0;
+  if (!locate_tile<W, RAGGED, TC, LT != 0>(a, sm.loc, loc, split)) return;
   const int kvh = loc.kvh, tile0 = loc.tile0;
   const int32_t fbeg = loc.fbeg, qs = loc.qs, qe = loc.qe, ps = loc.ps, pe = loc.pe;
 
@@ -1280,10 +1329,20 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
   const int64_t tile_end = kv_len - qo_len + (int)((uint32_t)f_last / (uint32_t)a.group) + 1;
   // (the page counts are wave-uniform; pinning them to SGPRs keeps the buffer
   // resources below scalar, with no waterfall loops around the loads)
-  const int npages = uni((int)((tile_end + 15) / 16));
+  int npages = uni((int)((tile_end + 15) / 16));
+  int blk0 = 0;
+  bool whole = true;
+  if constexpr (SPLIT) {
+    // this workgroup's share of the blocks: [blk0, blk0 + npages)
+    const int parts = tile_splits(npages, a.splits), n = npages;
+    if (split >= parts) return;
+    whole = parts == 1;
+    blk0 = (int)((int64_t)n * split / parts);
+    npages = (int)((int64_t)n * (split + 1) / parts) - blk0;
+  }
   // (SH: every wave walks every block; otherwise wave w takes blocks w, w + W, ...)
   const int mine = SH ? npages : uni(npages > wave ? (npages - wave + W - 1) / W : 0);
-  auto blk = [&](int i) { return SH ? i : wave + W * i; };
+  auto blk = [&](int i) { return SH ? i : SPLIT ? blk0 + wave + W * i : wave + W * i; };
 
   // Every page index of the request is checked (the reference rejects the
   // whole request; the verdict is read after the stream) and each wave takes
@@ -1309,7 +1368,10 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     }
   }
 
-  PrefillWave w{a, sm.qfrag[(SH && !LT) ? wave : 0], lane, col, quad, kvh};
+  constexpr bool KR = SPLIT;
+  __shared__ __align__(16) uint8_t ktile[KR ? W : 1][KR ? 16 * kKRowBytes : 16];
+  PrefillWave<KR> w{a, sm.qfrag[(SH && !LT) ? wave : 0], ktile[KR ? wave : 0],
+                    lane, col, quad, kvh};
   w.end_col = colv ? kv_len - qo_len + qi + 1 : 0;
   w.reset();
   // Long tiles: this lane's column of each of the wave's tiles.
@@ -1518,7 +1580,13 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     sm.m[wave][col] = w.m_run;
     sm.l[wave][col] = l_tot;
   }
-  if (block_or(bad, sm.bad)) return;
+  const bool refused = block_or(bad, sm.bad);
+  if constexpr (SPLIT) {
+    if (refused && !whole && wave == 0 && quad == 0)  // the merge keeps the sentinels
+      a.states[(((int64_t)split * a.row_tiles + loc.rank) * a.hkv + kvh) * 16 * kSplitState +
+               col * kSplitState + 1] = -1.0f;
+  }
+  if (refused) return;
   float M = -INFINITY;
 #pragma unroll
   for (int wv = 0; wv < W; ++wv) M = fmaxf(M, sm.m[wv][col]);
@@ -1545,6 +1613,26 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
       if (s > 1 || h == 0) __syncthreads();
     }
   }
+  if constexpr (SPLIT) {
+    if (!whole) {
+      if (wave != 0) return;
+      float *st = a.states + ((((int64_t)split * a.row_tiles + loc.rank) * a.hkv + kvh) * 16 + col) *
+                                 kSplitState;
+      float l = 0.0f;  // (a column that sees nothing of this share weighs nothing)
+#pragma unroll
+      for (int wv = 0; wv < W; ++wv)
+        l = fmaf(sm.l[wv][col], M == -INFINITY ? 0.0f : fast_exp2(sm.m[wv][col] - M), l);
+      // acc[e][i] = O[column][32 quad + 8 i + e]
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          *reinterpret_cast<f32x4 *>(st + 4 + 32 * quad + 8 * i + e) =
+              f32x4{w.acc[e][i], w.acc[e + 1][i], w.acc[e + 2][i], w.acc[e + 3][i]};
+      if (quad == 0) *reinterpret_cast<f32x2 *>(st) = f32x2{M, l};
+      return;
+    }
+  }
   if (wave != 0 || !colv) return;
   float L = 0.0f;
 #pragma unroll
@@ -1561,6 +1649,64 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     *reinterpret_cast<u32x4 *>(orow + r4 * 8) = o;
   }
   if (quad == 0) a.lse[row_head] = M + __log2f(L);
+}
+
+// Combines the states of the split row tiles: one workgroup per (tile,
+// kv-head), one wave per column, two dims per lane, all states of a column in
+// one round trip.  Tiles that were not split are done.
+template <bool RAGGED>
+__global__ __launch_bounds__(16 * 64) void prefill_split_merge_kernel(PrefillArgs a) {
+  __shared__ LocateSmem<16> sm;
+  const int lane = threadIdx.x & 63;
+  const int col = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  TileLoc loc;
+  if (!locate_tile<16, RAGGED, 16, false>(a, sm, loc)) return;
+  const int32_t ps = loc.ps, pe = loc.pe;
+  int64_t kv_len = pe - ps;
+  if constexpr (!RAGGED) {
+    if (ps < 0 || pe <= ps || pe > loc.ipB || loc.tl < 1 || loc.tl > a.page_rows) return;
+    kv_len = (int64_t)(pe - ps - 1) * a.page_rows + loc.tl;
+  }
+  const int qo_len = loc.qe - loc.qs;
+  if ((int64_t)qo_len > kv_len) return;
+  const int fcols = qo_len * a.group, f0 = loc.fbeg + loc.tile0 * 16;
+  const int64_t end =
+      kv_len - qo_len + (int)((uint32_t)min(f0 + 15, fcols - 1) / (uint32_t)a.group) + 1;
+  const int parts = tile_splits(uni((int)((end + 15) / 16)), a.splits);
+  const int f = f0 + col;
+  if (parts == 1 || f >= fcols) return;
+  const float *st = a.states + (((int64_t)loc.rank * a.hkv + loc.kvh) * 16 + col) * kSplitState;
+  const int64_t step = (int64_t)a.row_tiles * a.hkv * 16 * kSplitState;
+  f32x2 ml[kMaxSplits], x[kMaxSplits];
+#pragma unroll
+  for (int s = 0; s < kMaxSplits; ++s) {
+    ml[s] = f32x2{-INFINITY, 0.0f};
+    x[s] = f32x2{0.0f, 0.0f};
+    if (s < parts) {
+      ml[s] = *reinterpret_cast<const f32x2 *>(st + s * step);
+      x[s] = *reinterpret_cast<const f32x2 *>(st + s * step + 4 + 2 * lane);
+    }
+  }
+  float M = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < kMaxSplits; ++s) M = fmaxf(M, ml[s][0]);
+  float L = 0.0f, o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+  for (int s = 0; s < kMaxSplits; ++s) {
+    if (s < parts) {
+      if (ml[s][1] < 0.0f) return;  // refused: the rows keep their sentinels
+      const float w = M == -INFINITY ? 0.0f : fast_exp2(ml[s][0] - M);
+      L = fmaf(ml[s][1], w, L);
+      o0 = fmaf(x[s][0], w, o0);
+      o1 = fmaf(x[s][1], w, o1);
+    }
+  }
+  const float inv = 1.0f / L, v_scale = a.kv_scales ? a.kv_scales[1] : 1.0f;
+  const int qi = (int)((uint32_t)f / (uint32_t)a.group);
+  const int64_t row = (int64_t)(loc.qs + qi) * a.hq + (int64_t)loc.kvh * a.group + (f - qi * a.group);
+  *reinterpret_cast<uint32_t *>(a.out + row * 128 + 2 * lane) =
+      bf16x2_pack(o0 * inv * v_scale, o1 * inv * v_scale);
+  if (lane == 0) a.lse[row] = M + __log2f(L);
 }
 
 // The pipelined long-tile kernels: paged (BF16 or FP8 pages, weights rounded
@@ -1853,6 +1999,12 @@ __global__ __launch_bounds__(W * 64, LT ? (W == 8 ? (LT == 1 ? 4 : 2) : 3) : kPr
   prefill_body<W, false, FP8, SH, LT>(a);
 }
 
+// Row tiles split over several workgroups (PrefillArgs::splits).
+template <bool RAGGED, bool FP8>
+__global__ __launch_bounds__(4 * 64, kPrefillWavesPerEu) void prefill_split_kernel(PrefillArgs a) {
+  prefill_body<4, RAGGED, FP8, false, 0, true>(a);
+}
+
 // Pipelined long tiles: two waves per SIMD, two workgroups of four waves or
 // one of eight per CU.
 template <int W, int NW, bool FP8>
@@ -1885,12 +2037,16 @@ struct loom_paged_prefill_plan {
   uint32_t tile_cols = 16;  // flattened columns per workgroup
   uint32_t long_groups = 1;  // long tiles: wave groups splitting the K/V blocks
   bool pipe = false;         // long tiles: the pipelined kernel (PipeWave)
+  bool split_ok = false;     // row tiles: may be split over several workgroups
+  int cus = 0;
   uint32_t tile_layer = 0;   // serpentine tile order layer (PrefillArgs::tile_layer)
   bool tile_interleave = false;  // PrefillArgs::tile_interleave
 };
 
 struct loom_ragged_prefill_plan {
   loom_ragged_prefill_plan_info_t info{};
+  bool split_ok = false;     // row tiles: may be split over several workgroups
+  int cus = 0;
   uint32_t tile_cols = 16;   // flattened columns per workgroup
   uint32_t long_groups = 1;  // long tiles: wave groups splitting the K/V blocks
   uint32_t tile_layer = 0;   // PrefillArgs::tile_layer
@@ -1977,6 +2133,72 @@ loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
   }
   *tile_cols = long_requests && grid64 >= LOOM_PREFILL_WIDE_MIN_GRID ? 64 : 16;
   return LOOM_OK;
+}
+
+// What carries a row-tile command: 0: the fragment-order kernel; 1: whole-row
+// K loads; more: that, with so many workgroups per tile.  `blocks`: 16-row
+// blocks of all requests (a bound); microseconds on GQA4 32/8, before | after.
+//  - Tiles of one request that share its K/V through L2 (four and more per
+//    kv-head) wait for the CU's load path once more than one workgroup runs on
+//    a CU: whole rows (8 x 32 rows over 8192 tokens 159 | 112, over 512 14.9 |
+//    12.4; 2 x 100 over 2048 41.5 | 29.3), and so do contexts of up to 256
+//    tokens, whose first blocks are most of the walk (r256 8.7 | 7.5).
+//  - Long BF16 contexts of many requests, at memory speed (16 x 8 rows over
+//    8192 121 | 112, over 4096 51 | 45.5; FP8 pages 41 | 47: not taken;
+//    ragged within the runs' difference: not taken).
+//  - Else the fragment order: with one workgroup per CU the stream is bound by
+//    what one CU keeps in flight (about 55 GB/s), and the turn through LDS
+//    adds 4-6 % (16 x 1 over 2048 23.4 | 25.9).
+//  - Few streams (requests x kv-heads) of long contexts leave most of the
+//    chip idle: shares of at least 32 blocks, up to two workgroups per CU
+//    (1 x 4 rows over 2048 22.7 | 14.9, over 8192 75 | 18, 8 x 4 FP8 over 8192
+//    76 | 39).  Past 3/8 of the CUs the unsplit streams already draw 5 TB/s
+//    (16 x 1 over 4096 51 | 63), and a share pays for the merge (4-5 us).
+constexpr uint64_t kRowsShortBlocks = 16, kRowsLongBlocks = 256, kSplitMinBlocks = 128;
+template <bool RAGGED, bool FP8>
+int row_splits(uint64_t blocks, const PrefillArgs &a, uint64_t grid, int cus) {
+  const uint64_t batch = a.batch > 0 ? a.batch : 1, chip = (uint64_t)cus;
+  const uint64_t avg = blocks / batch, streams = batch * a.hkv;
+  // (a request's last tile is about half full)
+  const uint64_t tiles =
+      std::max<uint64_t>(batch, (uint64_t)a.nnz * a.group / 16 + batch / 2) * a.hkv;
+  if (tiles >= 4 * streams && (2 * tiles >= 3 * chip || avg <= kRowsShortBlocks)) return 1;
+  if (!RAGGED && !FP8 && tiles >= chip && 2 * streams >= chip && avg >= kRowsLongBlocks) return 1;
+  if (avg < kSplitMinBlocks || 8 * streams > 3 * chip ||
+      (4 * streams > chip && avg < kRowsLongBlocks))
+    return 0;
+  int s = kMaxSplits;
+  while (s > 1 && ((uint64_t)s * 32 > avg || grid * s > 2 * chip)) s /= 2;
+  return s >= 4 || (s == 2 && avg >= kRowsLongBlocks) ? s : 0;
+}
+
+// Runs a row-tile command split over several workgroups per tile, its states
+// in the queue's scratch; false: not worth it, or no scratch (a captured
+// stream without a reservation, no memory), and nothing was launched.
+template <bool RAGGED, bool FP8>
+bool launch_split(loom_command_scope_t *scope, PrefillArgs a, uint64_t blocks, uint64_t grid,
+                  int cus, hipError_t *e) {
+  const int splits = row_splits<RAGGED, FP8>(blocks, a, grid, cus);
+  if (splits < 1) return false;
+  uint8_t *ws = nullptr;
+  const uint64_t bytes = (uint64_t)splits * grid * 16 * kSplitState * 4;
+  if (splits > 1 &&
+      loom::queue_workspace(scope->queue, bytes, false, &ws, nullptr) != LOOM_OK) {
+    (void)hipGetLastError();
+    return false;
+  }
+  a.splits = splits;
+  a.states = (float *)ws;
+  hipStream_t stream = scope->queue->stream;
+  hipLaunchKernelGGL((prefill_split_kernel<RAGGED, FP8>), dim3((unsigned)(grid * splits)), dim3(256),
+                     0, stream, a);
+  *e = hipGetLastError();
+  if (*e == hipSuccess && splits > 1) {
+    hipLaunchKernelGGL(prefill_split_merge_kernel<RAGGED>, dim3((unsigned)grid), dim3(1024), 0,
+                       stream, a);
+    *e = hipGetLastError();
+  }
+  return true;
 }
 
 // The kernel of a paged plan.
@@ -2142,6 +2364,9 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
   p->tile_layer = long_tile && hkv_n > 0 && cus >= hkv_n && grid <= cus * resident
                       ? (uint32_t)(cus / hkv_n) : 0;
 
+  // (a page-index capacity says nothing about the contexts' lengths)
+  p->split_ok = p->info.algorithm == LOOM_PAGED_PREFILL_ROW_TILE && opt.waves == 0 && opt.flags == 0;
+  p->cus = provider->dev.cus;
   p->info.waves = waves;
   p->info.row_tiles = tiles;
   p->info.block_threads = 64 * (long_tile ? long_waves : p->info.waves);
@@ -2237,8 +2462,16 @@ loom_status_t loom_paged_prefill_enqueue(const loom_paged_prefill_plan_t *plan,
   a.blocks_lg = page_rows == 64 ? 2 : page_rows == 32 ? 1 : 0;
   a.tile_layer = (int32_t)plan->tile_layer;
   a.tile_interleave = plan->tile_interleave ? 1 : 0;
+  a.row_tiles = (int32_t)plan->info.row_tiles;
   hipStream_t stream = scope->queue->stream;
   const dim3 grid((unsigned)plan->info.grid_blocks), block(plan->info.block_threads);
+  if (plan->split_ok) {
+    const uint64_t blocks = (uint64_t)a.n_indices << a.blocks_lg;
+    hipError_t e = hipSuccess;
+    if (fp8 ? launch_split<false, true>(scope, a, blocks, plan->info.grid_blocks, plan->cus, &e)
+            : launch_split<false, false>(scope, a, blocks, plan->info.grid_blocks, plan->cus, &e))
+      return loom::record_launch(scope, e, err);
+  }
   if (fp8)
     launch_paged<true>(*plan, grid, block, stream, a);
   else
@@ -2299,6 +2532,8 @@ loom_status_t loom_prefill_provider_plan_bf16_ragged(
     p->tile_interleave = b <= 16 && (b >= 3 || (b == 2 && grid > 2 * cus * resident));
     p->tile_layer = hkv_n > 0 && cus >= hkv_n && grid <= cus * resident ? (uint32_t)(cus / hkv_n) : 0;
   }
+  p->split_ok = p->info.algorithm == LOOM_PAGED_PREFILL_ROW_TILE && opt.waves == 0 && opt.flags == 0;
+  p->cus = provider->dev.cus;
   p->info.waves = waves;
   p->info.row_tiles = tiles;
   p->info.block_threads = 64 * (long_tile ? tile_cols / 32 * p->long_groups : p->info.waves);
@@ -2370,6 +2605,12 @@ loom_status_t loom_ragged_prefill_enqueue(const loom_ragged_prefill_plan_t *plan
   const dim3 grid((unsigned)plan->info.grid_blocks), block(plan->info.block_threads);
   a.tile_layer = (int32_t)plan->tile_layer;
   a.tile_interleave = plan->tile_interleave ? 1 : 0;
+  a.row_tiles = (int32_t)plan->info.row_tiles;
+  if (plan->split_ok) {
+    hipError_t e = hipSuccess;
+    if (launch_split<true, false>(scope, a, s.nnz_kv / 16, plan->info.grid_blocks, plan->cus, &e))
+      return loom::record_launch(scope, e, err);
+  }
   switch (plan->info.waves) {
     case 4:
       if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && plan->tile_cols == 128 &&
