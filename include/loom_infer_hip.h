@@ -341,7 +341,10 @@ void loom_command_queue_free(loom_command_queue_t *queue);
  * split-KV states in a device buffer owned by the queue; this allocates it
  * ahead of the first command (`scratch_bytes` = a decode plan's
  * workspace_bytes) so that those enqueues allocate nothing, which is required
- * when they are captured.  `zeroed_bytes` (an append plan's workspace_bytes)
+ * when they are captured.  Direct single decode and row-tile prefill keep the
+ * states of their shares there too (16 * 528 bytes per share of a tile and
+ * kv-head); where the scratch does not hold them and cannot grow (a capture)
+ * they run unshared, with the same results up to summation order.  `zeroed_bytes` (an append plan's workspace_bytes)
  * is already held from queue creation; asking for more than that fails with
  * LOOM_ENQ_WORKSPACE_NOT_RESERVED.  Buffers only grow; they are freed with the
  * queue (or with the graph that captured its commands). */
@@ -693,7 +696,10 @@ typedef enum loom_paged_prefill_algorithm {
   /* One workgroup of `waves` waves per (request, kv-head, tile of 16
    * flattened (query row, group head) pairs).  The waves split the tile's
    * causal page range; per page, S = K·Qᵀ and O += P·V both run on MFMA, and
-   * the wave states merge in LDS.  No workspace. */
+   * the wave states merge in LDS.  No workspace operand; with the default
+   * `waves` a few rows over long contexts are shared by up to 16 workgroups
+   * per tile, their states in the queue's scratch (see
+   * loom_command_queue_reserve_workspace). */
   LOOM_PAGED_PREFILL_ROW_TILE = 1,
   /* For long prompts: one workgroup of four waves per (request, kv-head, tile
    * of 64 flattened pairs), one 16-column tile per wave.  Every wave walks the
@@ -702,15 +708,14 @@ typedef enum loom_paged_prefill_algorithm {
    * quarter of the L2 bytes per column that ROW_TILE reads.  No cross-wave
    * merge.  No workspace. */
   LOOM_PAGED_PREFILL_WIDE_TILE = 2,
-  /* Long prompts on BF16 or FP8 pages (paged prefill only): WIDE_TILE's
+  /* Long prompts, paged (BF16 or FP8 pages) or ragged: WIDE_TILE's
    * columns and page walk with 32-token blocks loaded straight into LDS, the
    * query fragments in registers and the softmax weights P rounded once to
    * BF16 for the P·V product (the normalizer is summed in FP32; within the
-   * attention tolerance of the f32 reference).  One or two 16-column query
-   * tiles per wave (64 or 128 columns per workgroup); plans whose grid fits
-   * one round of two workgroups per CU (and, with one tile per wave, requests
-   * averaging 1024 rows or more) run two groups of four waves that split the
-   * K/V blocks and merge in LDS (block_threads 512).  No workspace. */
+   * attention tolerance of the f32 reference; ragged: a BF16 high part and a
+   * residual).  64 or 128 columns per workgroup; plans whose grid leaves room
+   * for it run two or four groups of waves that split the K/V blocks and merge
+   * in LDS (block_threads 512).  No workspace. */
   LOOM_PAGED_PREFILL_LONG_TILE = 3
 } loom_paged_prefill_algorithm_t;
 

@@ -64,7 +64,7 @@ struct loom_command_queue {
   bool active = false;  // a scope or completion borrows the queue (Rust's &mut)
   // Device workspaces owned by the queue for the enqueue forms that take the
   // reference's argument structs (no workspace operand).  `scratch` holds
-  // split-KV states (no initialisation needed; grown on demand outside
+  // split-KV states of decode, single decode and row-tile prefill (no initialisation needed; grown on demand outside
   // stream capture, or reserved ahead).  `zeroed` holds the append
   // validation state: allocated and zero-filled when the queue is created
   // (its size is the same for every append plan), it carries the append

@@ -32,7 +32,11 @@
 // the whole causal block range, each block loaded once per workgroup (a
 // quarter per wave) into an LDS ring and read back by all four, so the L2
 // bytes per column fall fourfold; each wave finishes its own tile (no merge).
-// No workspace and one launch; the grid depends only on the plan.
+// Long tiles: see PipeWave and LongWave below.
+// Row tiles with many tiles per request load K as whole rows and turn it
+// through LDS; few rows over long contexts are shared by several workgroups
+// per tile, whose states a second launch merges (row_splits).  Otherwise no
+// workspace and one launch; the grid depends only on the plan.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
