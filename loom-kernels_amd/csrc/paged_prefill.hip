@@ -1728,6 +1728,7 @@ template <int W, int NW, bool RAGGED, bool FP8>
 __device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
   constexpr int G = W / NW;
   constexpr int TC = 32 * NW;  // flattened columns per workgroup
+  constexpr int kOutRow = 256 + 16;  // bytes of a row of O in LDS
   using Wave = PipeWave<NW, FP8, RAGGED, G>;
   // FP8 pages: K's scale folds into the score scale, V's into the output.
   PrefillArgs a = args;
@@ -1737,11 +1738,13 @@ __device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
     v_scale = a.kv_scales[1];
   }
   __shared__ PipeSmem<W, NW> sm;
-  // the groups' rings (several groups: also the merge staging of their column
-  // states, 64 floats per lane)
+  // the groups' rings, and after the walk the merge staging of several groups'
+  // column states (64 floats per lane) and the staging of O (32 rows per wave;
+  // FP8 pages: larger than one group's ring)
   constexpr int kRingBytes = G * Wave::kSlots * Wave::kSlotBytes;
   constexpr int kMergeBytes = G > 1 ? W * 64 * 64 * 4 : 0;
-  __shared__ __align__(16) uint8_t lring[kRingBytes > kMergeBytes ? kRingBytes : kMergeBytes];
+  constexpr int kOutBytes = W * 32 * kOutRow;
+  __shared__ __align__(16) uint8_t lring[std::max({kRingBytes, kMergeBytes, kOutBytes})];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, quad = lane >> 4;
@@ -1919,6 +1922,7 @@ __device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
     // dims that other groups finish to the ring's LDS (all waves are past
     // their last ring read: block_or's barrier), and group g finishes dims
     // 128 g / G .. of its columns.
+    static_assert(W * 2 * 8 * 64 * sizeof(f32x4) <= sizeof(lring), "merge staging");
     f32x4 *xs = reinterpret_cast<f32x4 *>(lring) + lane;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -1954,11 +1958,12 @@ __device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
   }
   // O through LDS (the ring is free; several groups: past a second barrier,
   // since other waves may still read the merge staging), each wave its own 32
-  // rows of 256 bytes at a stride of 272: whole rows then go out 16 bytes per
-  // lane (18 cycles of the CU's store path per KB; 8-byte pieces of 16 rows
+  // rows of 256 bytes at a stride of kOutRow: whole rows then go out 16 bytes
+  // per lane (18 cycles of the CU's store path per KB; 8-byte pieces of 16 rows
   // per instruction took 64, 2 us per workgroup of four waves).
   if constexpr (G > 1) __syncthreads();
-  uint8_t *ot = lring + wave * 32 * 272;
+  static_assert(W * 32 * kOutRow <= sizeof(lring), "O staging");
+  uint8_t *ot = lring + wave * 32 * kOutRow;
   int row_head[2];  // output row of each tile's column, -1: none
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
@@ -1968,7 +1973,7 @@ __device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
       if (e / kOwn == grp)
-        *reinterpret_cast<u32x2 *>(ot + (16 * t + col) * 272 + 32 * e + 8 * quad) =
+        *reinterpret_cast<u32x2 *>(ot + (16 * t + col) * kOutRow + 32 * e + 8 * quad) =
             u32x2{bf16x2_pack(lw.acc[t][e][0] * inv * v_scale, lw.acc[t][e][1] * inv * v_scale),
                   bf16x2_pack(lw.acc[t][e][2] * inv * v_scale, lw.acc[t][e][3] * inv * v_scale)};
     if (quad == 0 && grp == 0 && colv_t[t]) a.lse[row_head[t]] = M[t] + __log2f(L[t]);
@@ -1984,7 +1989,7 @@ __device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
     const int rh = r < 16 ? rh0 : rh1;
     if (rh >= 0)
       *reinterpret_cast<u32x4 *>(a.out + (int64_t)rh * 128 + unit * 8) =
-          *reinterpret_cast<const u32x4 *>(ot + r * 272 + unit * 16);
+          *reinterpret_cast<const u32x4 *>(ot + r * kOutRow + unit * 16);
   }
 }
 

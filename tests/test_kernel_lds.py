@@ -1,0 +1,66 @@
+"""CPU test of the built kernels' LDS: the metadata of the library's gfx950 code
+objects states each kernel's static LDS, which has to hold what its workgroup
+stages there."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+from conftest import PKG
+
+LIB = os.path.join(PKG, "lib", "libloom_infer_hip.so")
+READELF = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
+
+
+def code_objects(blob):
+    """The gfx950 ELF images of the offload bundles in `blob`."""
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    at = blob.find(magic)
+    while at >= 0:
+        (n,) = struct.unpack_from("<Q", blob, at + len(magic))
+        p = at + len(magic) + 8
+        for _ in range(n):
+            off, size, width = struct.unpack_from("<QQQ", blob, p)
+            triple = blob[p + 24:p + 24 + width]
+            p += 24 + width
+            if b"gfx950" in triple:
+                yield blob[at + off:at + off + size]
+        at = blob.find(magic, at + 1)
+
+
+@pytest.fixture(scope="module")
+def lds(tmp_path_factory):
+    """Kernel symbol -> bytes of static LDS."""
+    if not os.path.exists(READELF):
+        pytest.skip("no llvm-readelf")
+    out = {}
+    for i, image in enumerate(code_objects(open(LIB, "rb").read())):
+        path = tmp_path_factory.mktemp("co") / f"{i}.elf"
+        path.write_bytes(image)
+        notes = subprocess.run([READELF, "--notes", str(path)], check=True, capture_output=True,
+                               text=True).stdout
+        for k in re.split(r"^\s+- \.agpr_count", notes, flags=re.M)[1:]:
+            name = re.search(r"^ {4}\.name:\s+(\S+)", k, flags=re.M).group(1)
+            out[name] = int(re.search(r"\.group_segment_fixed_size:\s+(\d+)", k).group(1))
+    return out
+
+
+def test_pipelined_tiles_hold_their_staging(lds):
+    """After its walk each wave of a pipelined long tile stages 32 rows of O, 272
+    bytes apart, beside the workgroup's column states (max and normalizer of 32
+    columns and a flag per wave) and each wave's 64 page indices."""
+    found = {}
+    for name, have in lds.items():
+        m = re.search(r"(paged|ragged)_prefill_pipe_kernelILi(\d)ELi(\d)E(?:Lb([01])E)?", name)
+        if not m:
+            continue
+        waves = int(m.group(2))
+        need = waves * (32 * 272 + 2 * 32 * 4 + 4 + 64 * 4)
+        if int(m.group(3)) < waves:  # several wave groups: the merge of their columns' states
+            need = max(need, waves * (64 * 64 * 4 + 2 * 32 * 4 + 4 + 64 * 4))
+        found[m.group(0)] = (have, need)
+    assert len(found) == 12
+    short = {k: v for k, v in found.items() if v[0] < v[1]}
+    assert not short, short
