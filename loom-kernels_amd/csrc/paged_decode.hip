@@ -34,6 +34,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -1179,6 +1180,10 @@ __global__ __launch_bounds__(kThreads, waves_per_eu<GT>()) void single_decode_sp
     w.store_q(qr);
   }
   w.reset();
+  // A partition may begin with tokens that all score -inf: from the lowest
+  // finite maximum they weigh nothing, where -inf - (-inf) would make its whole
+  // state NaN.  (One with no other token stores the empty state.)
+  w.m_run = -FLT_MAX;
   const int nb = (int)((end - start + 15) / 16);
   auto tok_of = [&](int i) { return token_elem(a, start + (int64_t)min(i, nb - 1) * 16); };
   auto rows_of = [&](int i) {
@@ -1197,7 +1202,7 @@ __global__ __launch_bounds__(kThreads, waves_per_eu<GT>()) void single_decode_sp
         *reinterpret_cast<float2 *>(st + 2 + quad * 32 + i * 8 + e) =
             float2{w.acc[e][i], w.acc[e + 1][i]};
     if (quad == 0) {
-      st[0] = w.m_run;
+      st[0] = w.m_run == -FLT_MAX ? -INFINITY : w.m_run;
       st[1] = l_tot;
     }
   }

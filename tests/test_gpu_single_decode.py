@@ -190,3 +190,23 @@ def test_direct_plan_around_its_partitions(L, oracle, kv_len, hq, hkv):
             compare_decode(oracle, bf16_host(o), le.cpu().numpy(), *ref)
             if reserve:
                 assert np.array_equal(bf16_host(o), out)
+
+
+@pytest.mark.parametrize("kv_len,partitions", [(1024, None), (4096, None), (200, 12)])
+@pytest.mark.parametrize("first,count", [(64, 48), (70, 100)])
+def test_tokens_that_score_minus_infinity(L, oracle, kv_len, partitions, first, count):
+    """A run of keys whose scores overflow to -inf weighs nothing, wherever it
+    lies in a partition (its start, its whole, its middle): the result is that
+    of the other tokens."""
+    hq, hkv = 8, 2
+    q, k, v = fixture(oracle, kv_len, hq, hkv, 0x1F00 + kv_len)
+    q.reshape(hq, 128)[:, 0] = oracle.bf16_from_f32(np.float32([4.0]))[0]
+    rows = k.reshape(kv_len, hkv * 128)
+    rows[first:first + count] = 0
+    rows.reshape(kv_len, hkv, 128)[first:first + count, :, 0] = \
+        oracle.bf16_from_f32(np.float32([-3.0e38]))[0]
+    kept = np.r_[0:first, first + count:kv_len]
+    ref = oracle.single_decode(oracle.single_spec(len(kept), hq, hkv), q, rows[kept].ravel(),
+                               v.reshape(kv_len, -1)[kept].ravel())
+    out, lse = run_single(L, L.Bf16SingleDecodeSpec(kv_len, hq, hkv), q, k, v, partitions)
+    compare_decode(oracle, out, lse, *ref)
