@@ -329,7 +329,8 @@ typedef struct loom_handle {
  * a hipStream_t owned by the caller (it must outlive the queue).  Beyond the
  * reference, the queue allocates its append validation workspace here (device
  * memory, zero-filled by a kernel on `stream`; fails with
- * LOOM_ENQ_WORKSPACE_NOT_RESERVED if `stream` is being captured) and four
+ * LOOM_ENQ_WORKSPACE_NOT_RESERVED if `stream` is being captured), 4.1 MiB for
+ * the states of shared commands (loom_command_queue_reserve_workspace) and four
  * device status words in pinned host memory, which kernels write when they
  * cannot finish a command as specified (see LOOM_CMD_DEVICE_STATUS). */
 loom_status_t loom_command_queue_new(void *hip_stream, uint64_t max_commands,
@@ -341,16 +342,21 @@ void loom_command_queue_free(loom_command_queue_t *queue);
  * split-KV states in a device buffer owned by the queue; this allocates it
  * ahead of the first command (`scratch_bytes` = a decode plan's
  * workspace_bytes) so that those enqueues allocate nothing, which is required
- * when they are captured.  Direct single decode and row-tile prefill keep the
- * states of their shares there too (16 * 528 bytes per share of a tile and
- * kv-head); where the scratch does not hold them and cannot grow (a capture)
- * they run unshared, with the same results up to summation order.  `zeroed_bytes` (an append plan's workspace_bytes)
+ * when they are captured.  `zeroed_bytes` (an append plan's workspace_bytes)
  * is already held from queue creation; asking for more than that fails with
  * LOOM_ENQ_WORKSPACE_NOT_RESERVED.  Buffers only grow; they are freed with the
- * queue (or with the graph that captured its commands). */
+ * queue (or with the graph that captured its commands).
+ *
+ * Direct single decode of 640 tokens or more and row-tile prefill of few rows
+ * over long contexts keep states in a third buffer of the queue, 4.1 MiB from
+ * its creation on: they need no reservation, eager or in a graph queue's
+ * capture.  (Captured by the caller into a graph of its own, on the queue's
+ * stream, they run as one kernel each without it.) */
 loom_status_t loom_command_queue_reserve_workspace(loom_command_queue_t *queue,
                                                    uint64_t scratch_bytes, uint64_t zeroed_bytes,
                                                    loom_error_t *err);
+/* Bytes of the queue's workspaces that its commands and reservations so far
+ * have taken. */
 uint64_t loom_command_queue_workspace_bytes(const loom_command_queue_t *queue);
 uint64_t loom_command_queue_max_commands(const loom_command_queue_t *queue);
 int loom_command_queue_is_poisoned(const loom_command_queue_t *queue);
@@ -698,7 +704,7 @@ typedef enum loom_paged_prefill_algorithm {
    * causal page range; per page, S = K·Qᵀ and O += P·V both run on MFMA, and
    * the wave states merge in LDS.  No workspace operand; with the default
    * `waves` a few rows over long contexts are shared by up to 16 workgroups
-   * per tile, their states in the queue's scratch (see
+   * per tile, their states in a buffer of the queue (see
    * loom_command_queue_reserve_workspace). */
   LOOM_PAGED_PREFILL_ROW_TILE = 1,
   /* For long prompts: one workgroup of four waves per (request, kv-head, tile

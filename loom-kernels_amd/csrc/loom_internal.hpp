@@ -64,8 +64,11 @@ struct loom_command_queue {
   bool active = false;  // a scope or completion borrows the queue (Rust's &mut)
   // Device workspaces owned by the queue for the enqueue forms that take the
   // reference's argument structs (no workspace operand).  `scratch` holds
-  // split-KV states of decode, single decode and row-tile prefill (no initialisation needed; grown on demand outside
-  // stream capture, or reserved ahead).  `zeroed` holds the append
+  // split-KV states of paged decode (no initialisation needed; grown on demand
+  // outside stream capture, or reserved ahead).  `shares` holds the states of
+  // direct single decode's partitions and of row-tile prefill's shares: both
+  // have a small bound (kShareBytes), so it is allocated with the queue and
+  // their enqueues allocate nothing.  `zeroed` holds the append
   // validation state: allocated and zero-filled when the queue is created
   // (its size is the same for every append plan), it carries the append
   // kernels' epoch from one command to the next; all zeros is a valid
@@ -75,6 +78,8 @@ struct loom_command_queue {
   // use it.
   uint8_t *scratch = nullptr;
   uint64_t scratch_bytes = 0;
+  uint8_t *shares = nullptr;
+  bool shares_used = false;  // by some command of this queue
   uint8_t *zeroed = nullptr;
   uint64_t zeroed_bytes = 0;
   std::vector<void *> retired;
@@ -125,6 +130,19 @@ hipError_t synchronize_stream_or_abort(hipStream_t stream);
 // buffer.
 loom_status_t queue_workspace(loom_command_queue *queue, uint64_t bytes, bool zeroed,
                               uint8_t **out, loom_error_t *err);
+
+// Bytes of loom_command_queue::shares, the most that any command takes: row
+// tiles' shares run at most two workgroups per CU (256 on gfx950), each with 16
+// column states of 132 floats; single decode's partitions at most 1024 waves of
+// up to 8 query heads, 130 floats each.
+constexpr uint64_t kShareBytes = 512 * 16 * 132 * 4;
+static_assert(1024 * 8 * kStateWidth * 4 <= kShareBytes, "single decode's partitions");
+// The queue's share states for a command of `bytes`, or null: the command then
+// runs unshared.  Null for more than kShareBytes, and while a caller captures
+// the queue's stream into a graph of its own: its replays are not ordered with
+// the queue's other commands, nor bound to its lifetime.  (A graph queue's
+// capture has the buffer of its private queue, which the graph owns.)
+uint8_t *queue_shares(loom_command_scope *scope, uint64_t bytes);
 
 // Device status words of a command queue (loom_command_queue::status_*).
 enum DeviceStatus : int {

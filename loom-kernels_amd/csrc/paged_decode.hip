@@ -1915,16 +1915,13 @@ loom_status_t loom_single_decode_enqueue(const loom_single_decode_plan_t *plan,
   hipStream_t stream = scope->queue->stream;
   const int64_t L = (int64_t)s.kv_len;
   if (plan->partitions > 1) {
-    // The partial states live in the queue's scratch.  Where it is missing and
-    // cannot be allocated (a captured stream without a reservation, no
-    // memory) the one-kernel form runs.
-    uint8_t *ws = nullptr;
+    // The partial states live in the queue's share states; where a command
+    // may not use them the one-kernel form runs.
     const uint64_t bytes = s.num_query_heads * plan->partitions * loom::kStateWidth * 4;
-    if (loom::queue_workspace(scope->queue, bytes, false, &ws, nullptr) == LOOM_OK)
+    if (uint8_t *ws = loom::queue_shares(scope, bytes))
       return loom::record_launch(
           scope, launch_split_k(plan->group_tile, a, L, (int)plan->partitions, (float *)ws, stream),
           err);
-    (void)hipGetLastError();
   }
   const dim3 g3((unsigned)(s.num_kv_heads * plan->group_tiles)), b3(kThreads);
   switch (plan->group_tile) {

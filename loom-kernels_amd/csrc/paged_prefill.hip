@@ -2182,8 +2182,8 @@ int row_splits(uint64_t blocks, const PrefillArgs &a, uint64_t grid, int cus) {
 }
 
 // Runs a row-tile command split over several workgroups per tile, its states
-// in the queue's scratch; false: not worth it, or no scratch (a captured
-// stream without a reservation, no memory), and nothing was launched.
+// in the queue's share states; false: not worth it, or the command may not use
+// them, and nothing was launched.
 template <bool RAGGED, bool FP8>
 bool launch_split(loom_command_scope_t *scope, PrefillArgs a, uint64_t blocks, uint64_t grid,
                   int cus, hipError_t *e) {
@@ -2191,11 +2191,7 @@ bool launch_split(loom_command_scope_t *scope, PrefillArgs a, uint64_t blocks, u
   if (splits < 1) return false;
   uint8_t *ws = nullptr;
   const uint64_t bytes = (uint64_t)splits * grid * 16 * kSplitState * 4;
-  if (splits > 1 &&
-      loom::queue_workspace(scope->queue, bytes, false, &ws, nullptr) != LOOM_OK) {
-    (void)hipGetLastError();
-    return false;
-  }
+  if (splits > 1 && !(ws = loom::queue_shares(scope, bytes))) return false;
   a.splits = splits;
   a.states = (float *)ws;
   hipStream_t stream = scope->queue->stream;

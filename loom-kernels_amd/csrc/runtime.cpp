@@ -143,6 +143,21 @@ loom_status_t queue_workspace(loom_command_queue *q, uint64_t bytes, bool zeroed
   return LOOM_OK;
 }
 
+uint8_t *queue_shares(loom_command_scope *scope, uint64_t bytes) {
+  loom_command_queue *q = scope->queue;
+  if (bytes > kShareBytes) return nullptr;
+  if (!scope->capturing) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(q->stream, &cap) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+  }
+  q->shares_used = true;
+  return q->shares;
+}
+
 uint32_t read_device_status(const loom_command_queue *q) {
   uint32_t bits = 0;
   if (!q || !q->status_host) return 0;
@@ -187,9 +202,10 @@ int32_t settle(loom_command_completion *c, int32_t *sync_error) {
 }
 
 
-// The queue's device status words (pinned, mapped host memory, zeroed) and its
-// append validation workspace (device memory, zero-filled by a kernel on the
-// queue's stream, so every later command on the queue sees it zero).
+// The queue's device status words (pinned, mapped host memory, zeroed), its
+// share states and its append validation workspace (device memory, zero-filled
+// by a kernel on the queue's stream, so every later command on the queue sees it
+// zero).
 loom_status_t init_queue_memory(loom_command_queue *q, loom_error_t *err) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   hipError_t e = hipStreamIsCapturing(q->stream, &cap);
@@ -201,12 +217,13 @@ loom_status_t init_queue_memory(loom_command_queue *q, loom_error_t *err) {
   int prev = 0;
   hipGetDevice(&prev);
   hipSetDevice(q->device);
-  void *h = nullptr, *d = nullptr, *w = nullptr;
+  void *h = nullptr, *d = nullptr, *w = nullptr, *sh = nullptr;
   e = hipHostMalloc(&h, 64, hipHostMallocMapped | hipHostMallocPortable);
   if (e == hipSuccess) {
     memset(h, 0, 64);
     e = hipHostGetDevicePointer(&d, h, 0);
   }
+  if (e == hipSuccess) e = hipMalloc(&sh, loom::kShareBytes);
   if (e == hipSuccess) e = hipMalloc(&w, ws_bytes);
   if (e == hipSuccess) {
     const uint64_t words = ws_bytes / 4;
@@ -218,6 +235,7 @@ loom_status_t init_queue_memory(loom_command_queue *q, loom_error_t *err) {
   hipSetDevice(prev);
   q->status_host = (uint32_t *)h;
   q->status_dev = (uint32_t *)d;
+  q->shares = (uint8_t *)sh;
   q->zeroed = (uint8_t *)w;
   q->zeroed_bytes = w ? ws_bytes : 0;
   if (e != hipSuccess) return fail(err, LOOM_CMD_DRIVER, "queue memory", 0, 0, 0, 0, 0.0, e);
@@ -270,7 +288,7 @@ void loom_command_queue_free(loom_command_queue_t *q) {
               "loom-infer-hip command queue synchronized after a stream error during drop: %s\n",
               hipGetErrorString(e));
   }
-  if (q->scratch || q->zeroed || !q->retired.empty()) {
+  if (q->scratch || q->shares || q->zeroed || !q->retired.empty()) {
     // Commands that used the workspaces may still run (their completion was
     // dropped unsettled only after it synchronized, but a caller may free the
     // queue with work outstanding on a stream it shares with others).
@@ -279,6 +297,7 @@ void loom_command_queue_free(loom_command_queue_t *q) {
     hipGetDevice(&prev);
     hipSetDevice(q->device);
     if (q->scratch) hipFree(q->scratch);
+    if (q->shares) hipFree(q->shares);
     if (q->zeroed) hipFree(q->zeroed);
     for (void *p : q->retired) hipFree(p);
     hipSetDevice(prev);
@@ -302,7 +321,7 @@ loom_status_t loom_command_queue_reserve_workspace(loom_command_queue_t *q,
 }
 
 uint64_t loom_command_queue_workspace_bytes(const loom_command_queue_t *q) {
-  return q ? q->scratch_bytes + q->zeroed_bytes : 0;
+  return q ? q->scratch_bytes + q->zeroed_bytes + (q->shares_used ? loom::kShareBytes : 0) : 0;
 }
 
 uint64_t loom_command_queue_max_commands(const loom_command_queue_t *q) {

@@ -1,9 +1,12 @@
 """GPU parity of the row tiles' dispatch: whole-row K loads (one workgroup per
-tile) and shares of a tile's blocks merged from the queue's scratch, against
+tile) and shares of a tile's blocks merged from the queue's buffer, against
 the fragment-order kernel on the same pages (a plan with `waves` given), at
 the sizes where they can go wrong: shares of unequal length, tiles too short
 to split beside split ones, columns that see nothing of a share, every page
-form, a rejected request, and captures with and without a reservation."""
+form, a rejected request, captures with and without a reservation, and
+enqueues beside another queue's capture."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -118,8 +121,8 @@ def test_ragged_rows_match_the_fragment_order(L, oracle, case):
 
 @pytest.mark.parametrize("reserved", [0, 1 << 24])
 def test_captured_rows_replay(L, oracle, reserved):
-    """Without a reservation a capture records the fragment-order kernel (it
-    may not allocate); with one, the shares and their merge."""
+    """A capture records the shares and their merge, with a reservation and
+    without one (their states need none)."""
     import torch
     case = CASES[1]
     kw, pool, _, qkv, meta = case_inputs(case, "bf16")
@@ -145,3 +148,110 @@ def test_captured_rows_replay(L, oracle, reserved):
         exec_.launch().wait()
         assert_close(oracle, [(bf16_host(out), lse.view(torch.int32).cpu().numpy()), there])
     exec_.into_bindings()
+
+
+def shared_commands(L, oracle):
+    """(plan, args of a binding set, capacity, outputs) of a row-tile prefill that
+    runs in shares and of a single decode that runs as partitions."""
+    import torch
+    kw, pool, _, qkv, meta = case_inputs(CASES[1], "bf16")
+    spec = L.Bf16PagedPrefillSpec(2, 7, pool, 32, 8, **kw)
+    sspec = L.Bf16SingleDecodeSpec(4096, 32, 4)
+    for plan, cls, dev, s in (
+            (L.PrefillProvider.load(0).plan_bf16_paged(spec), L.Bf16PagedPrefillArgs,
+             qkv + [to_dev_i32(x) for x in meta], spec),
+            (L.DecodeProvider.load(0).plan_bf16(sspec), L.Bf16SingleDecodeArgs,
+             [torch.randn(n * 128, device="cuda").to(torch.bfloat16)
+              for n in (32, 4096 * 4, 4096 * 4)], sspec)):
+        outs = (nan_bf16(s.output_numel),
+                torch.full((s.lse_numel,), float("nan"), dtype=torch.float32, device="cuda"))
+
+        def args(b, cls=cls, dev=dev, outs=outs):
+            return cls(*[b.bind_read(x) for x in dev], *[b.bind_read_write(x).write() for x in outs])
+
+        yield plan, args, len(dev) + 2, outs
+
+
+def test_shared_commands_allocate_nothing(L, oracle):
+    """The states of shared commands live in a buffer that the queue has from its
+    creation on: the first enqueue on a fresh queue takes no device memory."""
+    import torch
+    for plan, args, n, outs in shared_commands(L, oracle):
+        queues = [L.CommandQueue(torch.cuda.Stream(), 1) for _ in range(4)]
+        gc.collect()  # (other tests' queues)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        for q in queues:
+            b = q.bindings(n)
+            a = args(b)
+            scope = q.begin(b)
+            plan.enqueue_into(scope, a)
+            scope.finish().wait()
+        assert torch.cuda.mem_get_info()[0] > free - (1 << 20)  # (each took 1 MiB or more)
+        assert not any(torch.isnan(x).any() for x in outs)
+
+
+def test_shared_commands_beside_a_capture(L, oracle):
+    """While this thread captures a graph, an eager shared command on another,
+    fresh queue runs and leaves the capture whole."""
+    import torch
+    cmds = list(shared_commands(L, oracle))
+    for plan, args, n, outs in cmds:
+        q = L.CommandQueue(torch.cuda.Stream(), 1)
+        gq = L.GraphQueue(0, 1)
+        torch.cuda.synchronize()
+        b, gb = q.bindings(n), gq.bindings(n)
+        held = [torch.empty_like(x) for x in outs]
+        a, ga = args(b), args(gb, outs=held)
+        pending = []
+
+        def record(scope):
+            plan.enqueue_into(scope, ga)
+            eager = q.begin(b)
+            plan.enqueue_into(eager, a)
+            pending.append(eager.finish())
+
+        graph = gq.capture(gb, record).instantiate()
+        pending[0].wait()
+        for _ in range(3):
+            for x in held:
+                x.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.launch().wait()
+            for x, y in zip(held, outs):
+                assert torch.equal(x, y) and not torch.isnan(x).any()
+        graph.into_bindings()
+
+
+def test_shared_commands_in_a_callers_capture(L, oracle):
+    """Captured by the caller into a graph of its own, whose replays the queue
+    does not order, a command keeps off the queue's buffer and runs unshared,
+    within the attention tolerance of the shared form."""
+    import torch
+    for plan, args, n, outs in shared_commands(L, oracle):
+        stream = torch.cuda.Stream()
+        eager, q = L.CommandQueue(stream, 1), L.CommandQueue(stream, 1)
+        b = eager.bindings(n)
+        a = args(b)
+        torch.cuda.synchronize()
+        scope = eager.begin(b)
+        plan.enqueue_into(scope, a)
+        scope.finish().wait()
+        held = [torch.empty_like(x) for x in outs]
+        b = q.bindings(n)
+        a = args(b, outs=held)
+        none = q.workspace_bytes
+        scope = q.begin(b)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+            plan.enqueue_into(scope, a)
+        scope.finish().wait()
+        assert q.workspace_bytes == none < eager.workspace_bytes
+        for _ in range(3):
+            for x in held:
+                x.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_close(oracle, [(bf16_host(o), l.view(torch.int32).cpu().numpy())
+                                  for o, l in (held, outs)])

@@ -159,11 +159,10 @@ def test_split_k_rejections_submit_nothing(L):
 @pytest.mark.parametrize("kv_len,hq,hkv", [(639, 32, 8), (640, 32, 8), (641, 8, 1),
                                            (1023, 28, 4), (2049, 32, 32), (8193, 32, 4)])
 def test_direct_plan_around_its_partitions(L, oracle, kv_len, hq, hkv):
-    """Direct plans of 640 tokens or more run as partitions and a merge in the
-    queue's scratch; a captured stream without a reservation keeps the one
-    kernel, and with one replays the two.  All within the attention gate of
-    the oracle; the two captures differ from the eager result by FP32 summation
-    order at most (one BF16 ulp, 2^-8 of values below 1)."""
+    """Direct plans of 640 tokens or more run as partitions and a merge in a
+    buffer of the queue, eager and captured, with a reservation (which they do
+    not need) and without one: all within the attention gate of the oracle, the
+    capture with a reservation bit-equal to the eager result."""
     import torch
     q, k, v = fixture(oracle, kv_len, hq, hkv, 0x5100 + kv_len)
     spec = L.Bf16SingleDecodeSpec(kv_len, hq, hkv)
