@@ -917,8 +917,14 @@ struct LongWave {
 //
 // acc[t][e][i] = O[column of tile t][dim 16 e + 4 quad + i].
 //
-// Normalizer past which a column's reference max is refreshed (see step()).
-constexpr float kRefreshNormalizer = 16777216.0f;
+// A column's reference lies kHeadroomLog2 above the largest score it was taken
+// from and moves when a lane's normalizer passes 1 (see step()), so a weight
+// never exceeds 1 and |O| stays below four times the largest |V|.  Along with it
+// move the columns past kNearRefresh, which would follow within a few blocks; a
+// column that has just moved is below it (9 * 2^-12).  Scores of unit variance
+// pass 1 only after some 80000 tokens (with 8 for 12, after 5000: 1% of an 8192
+// row prompt), and V's smallest normal values keep 11 bits of their products.
+constexpr float kHeadroomLog2 = 12.0f, kNearRefresh = 0.0625f;
 
 // HL: P enters the product as a BF16 high part and a BF16 residual (two MFMAs
 // per block of V), so the weights carry 16 significant bits and the
@@ -930,7 +936,7 @@ struct PipeWave {
   int lane, col, quad;
   int64_t end_col[2];  // causal end (exclusive) of the lane's column of each tile, 0 if unused
   int64_t full_end;    // smallest causal end of the wave's valid columns
-  float nmax[2];       // negated reference max (log2 domain, scaled); +inf: none yet
+  float nmax[2];       // negated reference (log2 domain, scaled); +inf: none yet
   float lsum[2];       // normalizer over the lane's quarter of the tokens
   f32x4 acc[2][8];
   u32x4 qf[2][4];      // B fragments of the query tiles
@@ -1139,12 +1145,12 @@ struct PipeWave {
       pin(nxt.s[0][x & 1], nxt.s[1][x & 1], l[x >> 2], p[x < 5 ? 2 * x + 7 : 15],
           p[x < 4 ? 2 * x + 8 : 15]);
     }
-    // The reference max of a column moves only when its normalizer passes
-    // kRefreshNormalizer or is not a number (no reference yet, or an
-    // overflow): BF16 and FP32 weights keep their relative precision at any
-    // magnitude, so a reference below the running max costs none, and the
-    // common step needs no max at all.  LSE = reference max + log2(normalizer).
-    if (__builtin_amdgcn_ballot_w64(!(l[0] <= kRefreshNormalizer && l[1] <= kRefreshNormalizer))) {
+    // The reference of a column moves only when its normalizer passes 1 or is
+    // not a number (no reference yet): BF16 and FP32 weights keep their relative
+    // precision at any magnitude, so a reference above the running max costs
+    // none, and the common step needs no max at all.  LSE = reference +
+    // log2(normalizer).
+    if (__builtin_amdgcn_ballot_w64(!(l[0] <= 1.0f && l[1] <= 1.0f))) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         float mx = fmaxf(cur.get(8 * t), cur.get(8 * t + 1));
@@ -1152,7 +1158,8 @@ struct PipeWave {
         for (int i = 2; i < 8; ++i) mx = fmaxf(mx, cur.get(8 * t + i));
         mx = quad_max(mx) * a.scale_log2;
         const float m_old = -nmax[t];
-        const float m_new = fmaxf(m_old, mx);
+        const bool move = !(quad_max_nan(l[t]) <= kNearRefresh);
+        const float m_new = move ? fmaxf(m_old, mx) + kHeadroomLog2 : m_old;
         const float m_use = m_new == -INFINITY ? 0.0f : m_new;  // nothing visible yet
         // (a column with nothing visible before has O = 0: nothing to rescale)
         const float al = fast_exp2(m_old - m_use);

@@ -177,3 +177,94 @@ def test_ragged_plans_match_row_tiles(L, oracle, shape):
     assert np.all(np.isfinite(o)) and np.abs(o - eo).max() <= 2.0 ** -6
     assert np.mean(o != eo) < 0.02
     assert np.abs(l - el).max() <= 1e-5
+
+
+def pipe_and_rows(L, oracle, plan, form, make_k, v_scale=1.0):
+    """((output, lse) of the plan's own algorithm, the 16-column algorithm's) on
+    the same inputs, outputs divided by v_scale; |q| and keys from
+    make_k(|normal|, token / kv_len)."""
+    import torch
+    from gpu_util import RaggedRunner, bf16_host, to_dev_i32
+    hq, hkv, qo_lens, kv_lens = plan[:4]
+    nnz, B = sum(qo_lens), len(qo_lens)
+    g = torch.Generator(device="cuda").manual_seed(nnz)
+    qo = np.concatenate([[0], np.cumsum(qo_lens)]).astype(np.int32)
+    at = np.concatenate([np.arange(n) / n for n in kv_lens])
+    n = len(at)
+    q = torch.randn(nnz * hq * 128, device="cuda", generator=g).abs().to(torch.bfloat16)
+    k, v = (torch.randn(n, hkv * 128, device="cuda", generator=g) for _ in range(2))
+    k = make_k(k.abs(), torch.from_numpy(at).to("cuda", torch.float32)[:, None])
+    # (below 4 one BF16 ulp, by which the rounding of the outputs may differ, is
+    # the gate's 2^-6; the weights' rounding moves them by less)
+    v = v.clamp(-3.75, 3.75) * v_scale
+    res = []
+    if form == "ragged":
+        kv = np.concatenate([[0], np.cumsum(kv_lens)]).astype(np.int32)
+        k, v = k.to(torch.bfloat16).flatten(), v.to(torch.bfloat16).flatten()
+        for tile in (0, 16):
+            r = RaggedRunner(L, B, nnz, n, hq, hkv, tile_cols=tile)
+            assert r.plan.algorithm == ("row_tile" if tile else "long_tile")
+            out, lse = r.run_dev(q, k, v, to_dev_i32(qo), to_dev_i32(kv))
+            res.append((bf16_host(out), lse.view(torch.int32).cpu().numpy()))
+    else:
+        pages = [(x + 15) // 16 for x in kv_lens]
+        pool = max(sum(pages) + 3, (2 * nnz + 15) // 16)
+        ip = np.concatenate([[0], np.cumsum(pages)]).astype(np.int32)
+        ix = np.random.default_rng(nnz).permutation(pool)[: ip[-1]].astype(np.int32)
+        last = np.array([x - (p - 1) * 16 for x, p in zip(kv_lens, pages)], np.int32)
+        row = np.concatenate([ix[ip[b] + np.arange(x) // 16].astype(np.int64) * 16 + np.arange(x) % 16
+                              for b, x in enumerate(kv_lens)])
+        pooled = []
+        for x in (k, v):
+            p = torch.zeros(pool * 16, hkv * 128, device="cuda")
+            p[torch.from_numpy(row).cuda()] = x
+            pooled.append(p.flatten())
+        kw, scales = {}, None
+        if form == "fp8":
+            kw, scales = {"kv_dtype": "fp8_e4m3"}, [0.8, 0.9]
+            k, v = (x.clamp(-440, 440).to(torch.float8_e4m3fn).view(torch.uint8) for x in pooled)
+        else:
+            k, v = (x.to(torch.bfloat16) for x in pooled)
+        p = L.PrefillProvider.load(0).plan_bf16_paged(
+            L.Bf16PagedPrefillSpec(B, nnz, pool, hq, hkv, **kw))
+        assert p.algorithm == "long_tile" and p.info.block_threads == plan[4]
+        res = paged_pair(L, B, nnz, pool, hq, hkv, q, k, v, qo, ip, ix, last, spec_kw=kw,
+                         scales=scales, tile="long")
+    # (powers of two: exact)
+    return [(oracle.bf16_from_f32(oracle.bf16_to_f32(o) / np.float32(v_scale)), l) for o, l in res]
+
+
+RANGE = [(p, "bf16") for p in PLANS] + [(p, "ragged") for p in RAGGED[:4]]
+
+
+@pytest.mark.parametrize("plan,form", RANGE + [(p, "fp8") for p in PLANS],
+                         ids=lambda x: x if isinstance(x, str) else f"{x[0]}x{x[1]}_{sum(x[2])}of{sum(x[3])}")
+def test_references_that_move_again_and_again(L, oracle, plan, form):
+    """Scores that rise by hundreds in the log2 domain along every context: each
+    form rescales O and the normalizers every few blocks."""
+    res = pipe_and_rows(L, oracle, plan, form, lambda k, at: k * at * 40)
+    assert float(np.nanmax(np.abs(res[1][1].view(np.float32)))) > 300
+    assert_close(oracle, res)
+
+
+@pytest.mark.parametrize("exponent", [115, -120])
+@pytest.mark.parametrize("plan,form", RANGE,
+                         ids=lambda x: x if isinstance(x, str) else f"{x[0]}x{x[1]}_{sum(x[2])}of{sum(x[3])}")
+def test_values_of_extreme_magnitude(L, oracle, plan, form, exponent):
+    """V of about 2^115 and 2^-120 under scores that rise by some 20 in the log2
+    domain: a weight is at most 1, so no sum of them with V leaves FP32's range
+    unless the result does, and small products keep BF16's precision."""
+    res = pipe_and_rows(L, oracle, plan, form, lambda k, at: k * at * 2, 2.0 ** exponent)
+    assert_close(oracle, res)
+
+
+@pytest.mark.parametrize("plan,form", RANGE,
+                         ids=lambda x: x if isinstance(x, str) else f"{x[0]}x{x[1]}_{sum(x[2])}of{sum(x[3])}")
+def test_runs_of_tokens_that_score_minus_infinity(L, oracle, plan, form):
+    """Whole blocks of keys whose scores overflow to -inf, the context's second
+    block among them, weigh nothing in every wave group."""
+    def keys(k, at):
+        k = k * 0.1
+        r = ((at > 0.07) & (at < 0.21)) | ((at > 0.4) & (at < 0.45))
+        return k.masked_fill(r, -3.0e38)
+    assert_close(oracle, pipe_and_rows(L, oracle, plan, form, keys))
