@@ -70,7 +70,8 @@ struct loom_command_queue {
   // have a small bound (kShareBytes), so it is allocated with the queue and
   // their enqueues allocate nothing.  `zeroed` holds the append
   // validation state: allocated and zero-filled when the queue is created
-  // (its size is the same for every append plan), it carries the append
+  // (its size is the same for every append plan, and it lies behind `shares` in
+  // one allocation), it carries the append
   // kernels' epoch from one command to the next; all zeros is a valid
   // starting state.  Commands on one queue are ordered on its one stream, so
   // they reuse the buffers without races.  A buffer that grows is retired,

@@ -1302,8 +1302,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
   TileLoc loc;
   const int split = SPLIT ? (int)(blockIdx.x / a.hkv) / a.row_tiles : 0;
   if (!locate_tile<W, RAGGED, TC, LT != 0>(a, sm.loc, loc, split)) return;
-  const int kvh = loc.kvh, tile0 = loc.tile0;
-  const int32_t fbeg = loc.fbeg, qs = loc.qs, qe = loc.qe, ps = loc.ps, pe = loc.pe;
+  const int kvh = loc.kvh, tile0 = uni(loc.tile0);
+  const int32_t fbeg = uni(loc.fbeg), qs = uni(loc.qs), qe = uni(loc.qe), ps = uni(loc.ps), pe = uni(loc.pe);
 
   // Per-request guards (paged: prefill.rs:316-342; ragged: applied in the
   // scan above, a failing request owns no tile).
@@ -1315,7 +1315,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     req_pages = (int)((kv_len + 15) / 16);
     tl = (int32_t)(kv_len - (int64_t)(req_pages - 1) * 16);
   } else {
-    tl = loc.tl;
+    tl = uni(loc.tl);
     if (ps < 0 || pe <= ps || pe > loc.ipB || tl < 1 || tl > a.page_rows) return;
     kv_len = (int64_t)(pe - ps - 1) * a.page_rows + tl;
     // 16-row blocks of the request and the valid rows of its last one

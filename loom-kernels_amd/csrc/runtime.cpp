@@ -203,9 +203,9 @@ int32_t settle(loom_command_completion *c, int32_t *sync_error) {
 
 
 // The queue's device status words (pinned, mapped host memory, zeroed), its
-// share states and its append validation workspace (device memory, zero-filled
-// by a kernel on the queue's stream, so every later command on the queue sees it
-// zero).
+// share states and its append validation workspace (zero-filled by a kernel on
+// the queue's stream, so every later command on the queue sees it zero), both in
+// one piece of device memory.
 loom_status_t init_queue_memory(loom_command_queue *q, loom_error_t *err) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   hipError_t e = hipStreamIsCapturing(q->stream, &cap);
@@ -217,26 +217,27 @@ loom_status_t init_queue_memory(loom_command_queue *q, loom_error_t *err) {
   int prev = 0;
   hipGetDevice(&prev);
   hipSetDevice(q->device);
-  void *h = nullptr, *d = nullptr, *w = nullptr, *sh = nullptr;
+  void *h = nullptr, *d = nullptr, *w = nullptr;
   e = hipHostMalloc(&h, 64, hipHostMallocMapped | hipHostMallocPortable);
   if (e == hipSuccess) {
     memset(h, 0, 64);
     e = hipHostGetDevicePointer(&d, h, 0);
   }
-  if (e == hipSuccess) e = hipMalloc(&sh, loom::kShareBytes);
-  if (e == hipSuccess) e = hipMalloc(&w, ws_bytes);
+  static_assert(loom::kShareBytes % 256 == 0, "the workspace behind it stays aligned");
+  if (e == hipSuccess) e = hipMalloc(&w, loom::kShareBytes + ws_bytes);
+  uint8_t *ws = w ? (uint8_t *)w + loom::kShareBytes : nullptr;
   if (e == hipSuccess) {
     const uint64_t words = ws_bytes / 4;
     hipLaunchKernelGGL(loom::zero_words_kernel,
                        dim3((unsigned)std::min<uint64_t>((words + 255) / 256, 1024)), dim3(256), 0,
-                       q->stream, (uint32_t *)w, words);
+                       q->stream, (uint32_t *)ws, words);
     e = hipGetLastError();
   }
   hipSetDevice(prev);
   q->status_host = (uint32_t *)h;
   q->status_dev = (uint32_t *)d;
-  q->shares = (uint8_t *)sh;
-  q->zeroed = (uint8_t *)w;
+  q->shares = (uint8_t *)w;
+  q->zeroed = ws;
   q->zeroed_bytes = w ? ws_bytes : 0;
   if (e != hipSuccess) return fail(err, LOOM_CMD_DRIVER, "queue memory", 0, 0, 0, 0, 0.0, e);
   return LOOM_OK;
@@ -288,7 +289,7 @@ void loom_command_queue_free(loom_command_queue_t *q) {
               "loom-infer-hip command queue synchronized after a stream error during drop: %s\n",
               hipGetErrorString(e));
   }
-  if (q->scratch || q->shares || q->zeroed || !q->retired.empty()) {
+  if (q->scratch || q->shares || !q->retired.empty()) {
     // Commands that used the workspaces may still run (their completion was
     // dropped unsettled only after it synchronized, but a caller may free the
     // queue with work outstanding on a stream it shares with others).
@@ -297,8 +298,7 @@ void loom_command_queue_free(loom_command_queue_t *q) {
     hipGetDevice(&prev);
     hipSetDevice(q->device);
     if (q->scratch) hipFree(q->scratch);
-    if (q->shares) hipFree(q->shares);
-    if (q->zeroed) hipFree(q->zeroed);
+    if (q->shares) hipFree(q->shares);  // and `zeroed` with it
     for (void *p : q->retired) hipFree(p);
     hipSetDevice(prev);
   }

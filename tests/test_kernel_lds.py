@@ -1,6 +1,6 @@
-"""CPU test of the built kernels' LDS: the metadata of the library's gfx950 code
-objects states each kernel's static LDS, which has to hold what its workgroup
-stages there."""
+"""CPU tests of the built kernels' resources: the metadata of the library's gfx950
+code objects states each kernel's static LDS, which has to hold what its workgroup
+stages there, and how many of its vector registers live in memory."""
 import os
 import re
 import struct
@@ -31,8 +31,8 @@ def code_objects(blob):
 
 
 @pytest.fixture(scope="module")
-def lds(tmp_path_factory):
-    """Kernel symbol -> bytes of static LDS."""
+def kernels(tmp_path_factory):
+    """Kernel symbol -> (bytes of static LDS, spilled vector registers)."""
     if not os.path.exists(READELF):
         pytest.skip("no llvm-readelf")
     out = {}
@@ -43,16 +43,17 @@ def lds(tmp_path_factory):
                                text=True).stdout
         for k in re.split(r"^\s+- \.agpr_count", notes, flags=re.M)[1:]:
             name = re.search(r"^ {4}\.name:\s+(\S+)", k, flags=re.M).group(1)
-            out[name] = int(re.search(r"\.group_segment_fixed_size:\s+(\d+)", k).group(1))
+            out[name] = tuple(int(re.search(r"\.%s:\s+(\d+)" % f, k).group(1))
+                              for f in ("group_segment_fixed_size", "vgpr_spill_count"))
     return out
 
 
-def test_pipelined_tiles_hold_their_staging(lds):
+def test_pipelined_tiles_hold_their_staging(kernels):
     """After its walk each wave of a pipelined long tile stages 32 rows of O, 272
     bytes apart, beside the workgroup's column states (max and normalizer of 32
     columns and a flag per wave) and each wave's 64 page indices."""
     found = {}
-    for name, have in lds.items():
+    for name, (have, _) in kernels.items():
         m = re.search(r"(paged|ragged)_prefill_pipe_kernelILi(\d)ELi(\d)E(?:Lb([01])E)?", name)
         if not m:
             continue
@@ -64,3 +65,9 @@ def test_pipelined_tiles_hold_their_staging(lds):
     assert len(found) == 12
     short = {k: v for k, v in found.items() if v[0] < v[1]}
     assert not short, short
+
+
+def test_no_kernel_spills_vector_registers(kernels):
+    """A spilled register of a tile's walk costs a memory round trip per block."""
+    assert len(kernels) > 50
+    assert {k: n for k, (_, n) in kernels.items() if n} == {}
