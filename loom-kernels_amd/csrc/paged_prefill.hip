@@ -2051,12 +2051,8 @@ struct loom_prefill_provider {
 struct loom_paged_prefill_plan {
   loom_paged_prefill_plan_info_t info{};
   uint32_t tile_cols = 16;  // flattened columns per workgroup
-  uint32_t long_groups = 1;  // long tiles: wave groups splitting the K/V blocks
-  bool pipe = false;         // long tiles: the pipelined kernel (PipeWave)
   bool split_ok = false;     // row tiles: may be split over several workgroups
   int cus = 0;
-  uint32_t tile_layer = 0;   // serpentine tile order layer (PrefillArgs::tile_layer)
-  bool tile_interleave = false;  // PrefillArgs::tile_interleave
 };
 
 struct loom_ragged_prefill_plan {
@@ -2157,8 +2153,7 @@ loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
 //  - Tiles of one request that share its K/V through L2 (four and more per
 //    kv-head) wait for the CU's load path once more than one workgroup runs on
 //    a CU: whole rows (8 x 32 rows over 8192 tokens 159 | 112, over 512 14.9 |
-//    12.4; 2 x 100 over 2048 41.5 | 29.3), and so do contexts of up to 256
-//    tokens, whose first blocks are most of the walk (r256 8.7 | 7.5).
+//    12.4; 2 x 100 over 2048 41.5 | 29.3; below, 3 x 13-24 over 220 7.1 | 7.7).
 //  - Long BF16 contexts of many requests, at memory speed (16 x 8 rows over
 //    8192 121 | 112, over 4096 51 | 45.5; FP8 pages 41 | 47: not taken;
 //    ragged within the runs' difference: not taken).
@@ -2168,9 +2163,12 @@ loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
 //  - Few streams (requests x kv-heads) of long contexts leave most of the
 //    chip idle: shares of at least 32 blocks, up to two workgroups per CU
 //    (1 x 4 rows over 2048 22.7 | 14.9, over 8192 75 | 18, 8 x 4 FP8 over 8192
-//    76 | 39).  Past 3/8 of the CUs the unsplit streams already draw 5 TB/s
-//    (16 x 1 over 4096 51 | 63), and a share pays for the merge (4-5 us).
-constexpr uint64_t kRowsShortBlocks = 16, kRowsLongBlocks = 256, kSplitMinBlocks = 128;
+//    76 | 39).  From 3/8 of the CUs on the unsplit streams already draw 5 TB/s
+//    (12 x 4 over 4096 41 | 50, 16 x 1 51 | 63), and a share pays for the merge
+//    (4-5 us).  Two shares of BF16 rows pay less: not for many requests whose
+//    tiles read K/V through different XCDs' L2 (kv-heads not a multiple of eight;
+//    16 x 6 rows over 4096 16/4 41 | 62, 4 x 42 over 4328 42 | 34).
+constexpr uint64_t kRowsLongBlocks = 256, kSplitMinBlocks = 128;
 template <bool RAGGED, bool FP8>
 int row_splits(uint64_t blocks, const PrefillArgs &a, uint64_t grid, int cus) {
   const uint64_t batch = a.batch > 0 ? a.batch : 1, chip = (uint64_t)cus;
@@ -2178,14 +2176,15 @@ int row_splits(uint64_t blocks, const PrefillArgs &a, uint64_t grid, int cus) {
   // (a request's last tile is about half full)
   const uint64_t tiles =
       std::max<uint64_t>(batch, (uint64_t)a.nnz * a.group / 16 + batch / 2) * a.hkv;
-  if (tiles >= 4 * streams && (2 * tiles >= 3 * chip || avg <= kRowsShortBlocks)) return 1;
+  if (tiles >= 4 * streams && 2 * tiles >= 3 * chip) return 1;
   if (!RAGGED && !FP8 && tiles >= chip && 2 * streams >= chip && avg >= kRowsLongBlocks) return 1;
-  if (avg < kSplitMinBlocks || 8 * streams > 3 * chip ||
+  if (avg < kSplitMinBlocks || 8 * streams >= 3 * chip ||
       (4 * streams > chip && avg < kRowsLongBlocks))
     return 0;
   int s = kMaxSplits;
   while (s > 1 && ((uint64_t)s * 32 > avg || grid * s > 2 * chip)) s /= 2;
-  return s >= 4 || (s == 2 && avg >= kRowsLongBlocks) ? s : 0;
+  const bool two = avg >= kRowsLongBlocks && (FP8 || a.hkv % 8 == 0 || 8 * streams < chip);
+  return s >= 4 || (s == 2 && two) ? s : 0;
 }
 
 // Runs a row-tile command split over several workgroups per tile, its states
@@ -2213,16 +2212,113 @@ bool launch_split(loom_command_scope_t *scope, PrefillArgs a, uint64_t blocks, u
   return true;
 }
 
+// How the long tiles of a paged command run.
+struct LongForm {
+  bool pipe;          // the pipelined kernel (PipeWave), else the plain one (LongWave)
+  uint32_t groups;    // wave groups splitting the K/V blocks
+  bool interleave;    // PrefillArgs::tile_interleave
+  uint32_t layer;     // serpentine tile order layer (PrefillArgs::tile_layer)
+  // waves per workgroup: column waves (pipelined: 32 columns each, else 16 or
+  // 32) times groups
+  uint32_t waves(uint32_t tile_cols) const { return (pipe ? tile_cols / 32 : 4) * groups; }
+};
+
+// The form for requests whose contexts hold `tokens` tokens in all (whole pages).
+// Microseconds on GQA4 32/8 and BF16 pages unless stated, one box; plain and pipe
+// are the kernels.
+//
+// 128 columns: the pipelined kernel, in two groups of four waves, where the grid
+// holds at most two workgroups per CU (1 x 2048 rows 53.7 plain / 48.5, 4 x 512
+// rows behind 2048-16384 tokens 473 / 384), and on FP8 pages, whose plain walk is
+// slower.  Larger BF16 grids: two pipelined workgroups per CU or three plain
+// ones.  The pipelined ones walk faster, but three rounds of them take what two
+// plain rounds take, and short contexts are all start and end:
+//  - Whole prompts leave light tiles for the second round: pipe from 400 tokens
+//    on up to 19/8 workgroups per CU (4 x 348-642 rows 27.8 / 24.7), 650 to five
+//    (8 x 733-1216 16/4 63.1 / 56.5; 16 x 233-397 16/4 24.6 / 29.5), but 1024
+//    just past three, a full round of plain ones (4 x 711-1047 28/4 43.4 / 45.5,
+//    4 x 1809-2553 16/4 118.9 / 100.0); one prompt at any size (5776 rows 282 /
+//    268), more requests not past five (8 x 1024 89.6 / 93.8).
+//  - Contexts of 2.5 tokens per row and more walk about equally long: pipe where
+//    its rounds are fewer, up to 19/8 workgroups per CU (11 x 162-249 rows behind
+//    2861 28/4 119 / 87 without interleaving) and from three to five (9 x 242-471
+//    behind 2333 32/32 161 / 133); between, plain (9 x 196-310 behind 2827 124 /
+//    144).
+//  - In between plain, but for 13/4 to 17/4 per CU (9 x 166-252 behind 408 64/8
+//    38.9 / 34.7).
+//
+// 64 columns (grids too small for 128): the pipelined kernel with two column
+// waves, in two groups (two workgroups per CU), or in four where the grid holds
+// at most one workgroup per CU, for contexts twice as long as the prompts (512
+// rows behind 15872 tokens 276 plain / 179 two groups / 150 four) and, in plans
+// whose pool has room for such contexts, for long prompts (1 x 1140 rows 28.2 /
+// 23.5, but 1 x 512 12.9 / 12.8 / 13.8, 2 x 512 16.0 / 16.6, 13 x 57-71 28/4 11.0 /
+// 11.8).  On grids of a second round its starts and ends show unless the
+// requests are long (12 x 100 rows 11.1 / 20.2, 6 x 200 12.1 / 21.0).  The plain
+// kernel in two groups of four waves where its grid fits one round of two such
+// workgroups per CU or the requests are long (two groups against one: 1 x 512
+// rows -6%, 1 x 1536 -10%, 2 x 512 +6%).
+LongForm long_form(const loom_paged_prefill_plan &p, uint64_t tokens) {
+  const auto &spec = p.info.spec;
+  const uint64_t cus = (uint64_t)p.cus, hkv = spec.num_kv_heads, b = spec.batch_size;
+  const uint64_t grid = p.info.grid_blocks, nnz = spec.nnz_qo;
+  const bool fp8 = spec.kv_dtype == LOOM_KV_DTYPE_FP8_E4M3;
+  const bool two_per_cu = grid <= 2 * cus, long_rows = nnz >= 1024 * b;
+  const bool prefix = 2 * tokens >= 5 * nnz;
+  const uint64_t page_rows = spec.page_size ? spec.page_size : loom::kPageSize;
+  LongForm f{};
+  if (p.tile_cols == 128) {
+    // workgroups that find a tile: every request's last tile is about half full
+    const uint64_t tiles = nnz * (spec.num_query_heads / hkv) / 128 * hkv + b * hkv / 2;
+    if (fp8 || two_per_cu)
+      f.pipe = true;
+    else if (8 * tokens < 9 * nnz)
+      f.pipe = tokens >= b * (8 * tiles <= 19 * cus                      ? 400
+                              : tiles > 3 * cus && 2 * tiles <= 7 * cus ? 1024
+                                                                        : 650) &&
+               (b == 1 || grid <= 5 * cus);
+    else if (prefix)
+      f.pipe = 8 * tiles <= 19 * cus || (tiles > 3 * cus && tiles <= 5 * cus);
+    else
+      f.pipe = 4 * tiles > 13 * cus && 4 * tiles <= 17 * cus;
+    f.groups = two_per_cu ? 2 : 1;
+  } else {
+    const bool roomy = spec.max_num_pages * page_rows >= 2 * nnz;
+    f.pipe = (tokens >= 2 * nnz || (roomy && nnz >= 768 * b)) && (two_per_cu || long_rows);
+    f.groups = f.pipe && grid <= cus ? 4 : two_per_cu || long_rows ? 2 : 1;
+  }
+  // Serpentine tile order when the whole grid is resident at once (two
+  // pipelined workgroups of four waves per CU, one of eight; plain: three of
+  // four waves, two of eight).  A second round is dispatched as CUs free up,
+  // where heaviest-first order balances better (1 x 1024 rows 28.6 -> 25.3, 2 x
+  // 512 18.5 -> 17.2, 8 x 256 20.1 -> 19.8; on grids of more than one round 1 x
+  // 2048 in two groups 58 -> 70, 1 x 4096 141 -> 147, 4 x 2048 153 -> 163).
+  const uint64_t resident = f.pipe ? (f.waves(p.tile_cols) == 8 ? 1 : 2) : f.groups == 2 ? 2 : 3;
+  f.layer = hkv > 0 && cus >= hkv && grid <= cus * resident ? (uint32_t)(cus / hkv) : 0;
+  // Requests' tiles interleaved by their distance from the request's end, so
+  // that every request's heaviest tiles are dispatched first (the search takes
+  // up to 64 requests): 3 x 512 rows -8% (FP8 -19%), 8 x 1024 -8 / -16%, 4 x 2048
+  // -4 / -7%, 16 x 512 0 / -6%; many short requests lost (32 x 256 +2%, 64 x 128
+  // +5%).  Two requests only on grids of more than six workgroups per CU (2 x
+  // 4096 0 / -12%): below, unequal ones lose up to a quarter (1838 and 4101 rows
+  // 28/4 155 -> 199).  Pipelined tiles behind long prefixes on BF16 pages, whose
+  // walks hardly differ, run request by request (11 x 193-381 rows behind
+  // 1816-5645 32/32 412 -> 310).
+  const bool by_request = f.pipe && !fp8 && !two_per_cu && p.tile_cols == 128 && prefix;
+  f.interleave = b <= 16 && (b >= 3 || (b == 2 && grid > 6 * cus)) && !by_request;
+  return f;
+}
+
 // The kernel of a paged plan.
 template <bool FP8>
-void launch_paged(const loom_paged_prefill_plan &p, dim3 grid, dim3 block, hipStream_t stream,
-                  const PrefillArgs &a) {
-  if (p.info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && p.pipe) {
-    if (p.tile_cols == 128 && p.long_groups == 2)
+void launch_paged(const loom_paged_prefill_plan &p, const LongForm &form, dim3 grid, dim3 block,
+                  hipStream_t stream, const PrefillArgs &a) {
+  if (p.info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE && form.pipe) {
+    if (p.tile_cols == 128 && form.groups == 2)
       hipLaunchKernelGGL((paged_prefill_pipe_kernel<8, 4, FP8>), grid, block, 0, stream, a);
     else if (p.tile_cols == 128)
       hipLaunchKernelGGL((paged_prefill_pipe_kernel<4, 4, FP8>), grid, block, 0, stream, a);
-    else if (p.long_groups == 4)
+    else if (form.groups == 4)
       hipLaunchKernelGGL((paged_prefill_pipe_kernel<8, 2, FP8>), grid, block, 0, stream, a);
     else
       hipLaunchKernelGGL((paged_prefill_pipe_kernel<4, 2, FP8>), grid, block, 0, stream, a);
@@ -2232,7 +2328,7 @@ void launch_paged(const loom_paged_prefill_plan &p, dim3 grid, dim3 block, hipSt
         hipLaunchKernelGGL((paged_prefill_kernel<4, false, true, 2>), grid, block, 0, stream, a);
         return;
       }
-    if (p.long_groups == 2)
+    if (form.groups == 2)
       hipLaunchKernelGGL((paged_prefill_kernel<8, FP8, true, 1>), grid, block, 0, stream, a);
     else
       hipLaunchKernelGGL((paged_prefill_kernel<4, FP8, true, 1>), grid, block, 0, stream, a);
@@ -2308,82 +2404,17 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
                       : tile_cols == 64 ? LOOM_PAGED_PREFILL_WIDE_TILE
                                         : LOOM_PAGED_PREFILL_ROW_TILE;
   p->tile_cols = tile_cols;
-  // The long tiles' kernel and wave groups.  Microseconds on GQA4 32/8, BF16,
-  // one box (plain: LongWave; pipe: PipeWave).
-  //
-  // 128 columns: the pipelined kernel, in two groups of four waves when the
-  // grid holds at most two workgroups per CU.  Its two workgroups per CU walk
-  // long ranges faster, but hide less of a workgroup's start and end than the
-  // plain kernel's three, so batches of requests whose grids run for more
-  // than about two rounds keep the plain kernel on BF16 pages (FP8 pages,
-  // whose plain walk is slower, do not).  plain / pipe: 1 x 2048 rows 53.7 /
-  // 48.5, 1 x 4096 139 / 134, 1 x 8192 513 / 502, 2 x 2048 89 / 76, 8 x 256
-  // 18.9 / 16.5, 8 x 512 40.8 / 38.9, 16 x 256 34.3 / 32.7; 8 x 1024 89.6 /
-  // 93.8, 16 x 512 67.8 / 75.6, 4 x 2048 146.5 / 147.5 (FP8 4 x 2048 157 /
-  // 147); 4 x 512 rows behind 2048-16384 tokens 473 / 384 (FP8 557 / 427).
-  //
-  // 64 columns (grids too small for 128), where the pool may hold contexts
-  // longer than the prompts: the pipelined kernel with two column waves, in
-  // two groups (two workgroups per CU), or in four where the grid holds at
-  // most one workgroup per CU.  plain / two groups / four: 1 x 512 rows 12.9 /
-  // 12.8 / 13.8, 1 x 1024 21.5 / 20.8 / 30.4, 1 x 1536 37.8 / 34.8 / 47.3, 2 x
-  // 512 16.0 / 16.6 / 16.6; 512 rows behind 15872 tokens 276 / 179 / 150.  On
-  // grids of a second round its starts and ends show unless the requests are
-  // long (12 x 100 rows 11.1 / 20.2, 6 x 200 12.1 / 21.0): the plain kernel.
-  // A pool that holds hardly more than the prompts keeps the plain kernel:
-  // two groups of four waves, halving the longest tiles' serial block walk,
-  // when the grid fits one round of two such workgroups per CU or the
-  // requests are long enough (1024 rows on average) that the heaviest tiles
-  // dominate (two groups against one: 1 x 512 rows -6%, 1 x 1536 -10%, 2 x 512
-  // +6%).
-  const uint64_t cus = provider->dev.cus, hkv_n = spec->num_kv_heads;
-  const bool two_per_cu = grid <= 2 * cus;
-  const bool fp8_pages = spec->kv_dtype == LOOM_KV_DTYPE_FP8_E4M3;
+  p->cus = provider->dev.cus;
   const uint64_t page_rows = spec->page_size ? spec->page_size : loom::kPageSize;
-  const bool roomy = spec->max_num_pages >= (2 * spec->nnz_qo + page_rows - 1) / page_rows;
-  if (long_tile && tile_cols == 128) {
-    p->pipe = fp8_pages || spec->batch_size < 3 || grid <= 5 * cus;
-    p->long_groups = two_per_cu ? 2 : 1;
-  } else if (long_tile && roomy && (two_per_cu || spec->nnz_qo >= 1024 * spec->batch_size)) {
-    p->pipe = true;
-    p->long_groups = grid <= cus ? 4 : 2;
-  } else if (long_tile) {
-    p->long_groups = two_per_cu || spec->nnz_qo >= 1024 * spec->batch_size ? 2 : 1;
-  }
-  // waves per workgroup: column waves (pipelined: 32 columns each, else 16 or
-  // 32) times groups
-  const uint32_t long_waves = (p->pipe ? tile_cols / 32 : 4) * p->long_groups;
-  // Serpentine tile order when the whole grid is resident at once (long
-  // tiles: three 4-wave workgroups per CU; two 8-wave ones of one tile per
-  // wave; one of two tiles per wave).  A second round is dispatched as CUs
-  // free up, where heaviest-first order balances better.  Measured (GQA4
-  // 32/8, BF16, same box): 1 x 1024 rows 28.6 -> 25.3 us, 2 x 512 18.5 ->
-  // 17.2, 1 x 3072 100.5 -> 98.0, 8 x 256 20.1 -> 19.8; on grids of more
-  // than one round 1 x 2048 (two tiles, two groups) 58 -> 70, 1 x 4096 141 ->
-  // 147, 4 x 2048 153 -> 163.
-  const uint64_t resident = p->pipe ? (long_waves == 8 ? 1 : 2) : p->long_groups == 2 ? 2 : 3;
-  // Requests' tiles interleaved by their distance from the request's end, so
-  // that every request's heaviest tiles are dispatched first (the kernel
-  // takes up to 64 requests, whose tile counts one wave holds).  Measured (GQA4
-  // 32/8, BF16 / FP8 pages, same box): 3 x 512 rows -8% / -19%, 4 x 512 -3% /
-  // -4%, 8 x 256 -3% / -6%, 8 x 1024 -8% / -16%, 4 x 2048 -4% / -7%, 16 x 512
-  // 0 / -6%, 2 x 4096 (more than two rounds) 0 / -12%; two requests on a grid
-  // of one or two rounds lost (2 x 512 +9% / +4%, 2 x 1024 +2% / +2%), and
-  // so did many short requests (32 x 256 +2%, 64 x 128 +5%).
-  const uint64_t b = spec->batch_size;
-  p->tile_interleave = long_tile && b <= 16 &&
-                       (b >= 3 || (b == 2 && grid > 2 * cus * resident));
-  p->tile_layer = long_tile && hkv_n > 0 && cus >= hkv_n && grid <= cus * resident
-                      ? (uint32_t)(cus / hkv_n) : 0;
-
   // (a page-index capacity says nothing about the contexts' lengths)
   p->split_ok = p->info.algorithm == LOOM_PAGED_PREFILL_ROW_TILE && opt.waves == 0 && opt.flags == 0;
-  p->cus = provider->dev.cus;
   p->info.waves = waves;
   p->info.row_tiles = tiles;
-  p->info.block_threads = 64 * (long_tile ? long_waves : p->info.waves);
   p->info.grid_blocks = grid;
   p->info.flags = opt.flags;
+  // (of the form that contexts filling the pool take)
+  p->info.block_threads =
+      64 * (long_tile ? long_form(*p, spec->max_num_pages * page_rows).waves(tile_cols) : waves);
   *out = p;
   return loom::ok(err);
 }
@@ -2472,11 +2503,17 @@ loom_status_t loom_paged_prefill_enqueue(const loom_paged_prefill_plan_t *plan,
   a.row_elems = hnd ? 128 : a.hkv * 128;
   a.page_rows = (int32_t)page_rows;
   a.blocks_lg = page_rows == 64 ? 2 : page_rows == 32 ? 1 : 0;
-  a.tile_layer = (int32_t)plan->tile_layer;
-  a.tile_interleave = plan->tile_interleave ? 1 : 0;
+  LongForm form{};
+  uint32_t threads = plan->info.block_threads;
+  if (plan->info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE) {
+    form = long_form(*plan, (uint64_t)a.n_indices * page_rows);
+    threads = 64 * form.waves(plan->tile_cols);
+  }
+  a.tile_layer = (int32_t)form.layer;
+  a.tile_interleave = form.interleave ? 1 : 0;
   a.row_tiles = (int32_t)plan->info.row_tiles;
   hipStream_t stream = scope->queue->stream;
-  const dim3 grid((unsigned)plan->info.grid_blocks), block(plan->info.block_threads);
+  const dim3 grid((unsigned)plan->info.grid_blocks), block(threads);
   if (plan->split_ok) {
     const uint64_t blocks = (uint64_t)a.n_indices << a.blocks_lg;
     hipError_t e = hipSuccess;
@@ -2485,9 +2522,9 @@ loom_status_t loom_paged_prefill_enqueue(const loom_paged_prefill_plan_t *plan,
       return loom::record_launch(scope, e, err);
   }
   if (fp8)
-    launch_paged<true>(*plan, grid, block, stream, a);
+    launch_paged<true>(*plan, form, grid, block, stream, a);
   else
-    launch_paged<false>(*plan, grid, block, stream, a);
+    launch_paged<false>(*plan, form, grid, block, stream, a);
   return loom::record_launch(scope, hipGetLastError(), err);
 }
 
@@ -2541,7 +2578,7 @@ loom_status_t loom_prefill_provider_plan_bf16_ragged(
     p->long_groups = tile_cols == 128 ? (grid <= 2 * cus ? 2 : 1) : (grid <= cus ? 4 : 2);
     const uint32_t long_waves = tile_cols / 32 * p->long_groups;
     const uint64_t resident = long_waves == 8 ? 1 : 2;
-    p->tile_interleave = b <= 16 && (b >= 3 || (b == 2 && grid > 2 * cus * resident));
+    p->tile_interleave = b <= 16 && (b >= 3 || (b == 2 && grid > 6 * cus));
     p->tile_layer = hkv_n > 0 && cus >= hkv_n && grid <= cus * resident ? (uint32_t)(cus / hkv_n) : 0;
   }
   p->split_ok = p->info.algorithm == LOOM_PAGED_PREFILL_ROW_TILE && opt.waves == 0 && opt.flags == 0;
