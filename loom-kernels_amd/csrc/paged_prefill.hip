@@ -2230,8 +2230,9 @@ struct LongForm {
 // 128 columns: the pipelined kernel, in two groups of four waves, where the grid
 // holds at most two workgroups per CU (1 x 2048 rows 53.7 plain / 48.5, 4 x 512
 // rows behind 2048-16384 tokens 473 / 384), and on FP8 pages, whose plain walk is
-// slower.  Larger BF16 grids: two pipelined workgroups per CU or three plain
-// ones.  The pipelined ones walk faster, but three rounds of them take what two
+// slower, unless requests of less than 420 tokens fill 9/4 to three workgroups
+// per CU (10 x 94-167 rows 64/8 20.6 / 22.3, 16 x 202-390 16/4 23.5 / 26.4).
+// Larger BF16 grids: two pipelined workgroups per CU or three plain ones.  The pipelined ones walk faster, but three rounds of them take what two
 // plain rounds take, and short contexts are all start and end:
 //  - Whole prompts leave light tiles for the second round: pipe from 400 tokens
 //    on up to 19/8 workgroups per CU (4 x 348-642 rows 27.8 / 24.7), 650 to five
@@ -2270,8 +2271,10 @@ LongForm long_form(const loom_paged_prefill_plan &p, uint64_t tokens) {
   if (p.tile_cols == 128) {
     // workgroups that find a tile: every request's last tile is about half full
     const uint64_t tiles = nnz * (spec.num_query_heads / hkv) / 128 * hkv + b * hkv / 2;
-    if (fp8 || two_per_cu)
+    if (two_per_cu)
       f.pipe = true;
+    else if (fp8)
+      f.pipe = 4 * tiles < 9 * cus || tiles > 3 * cus || tokens >= 420 * b;
     else if (8 * tokens < 9 * nnz)
       f.pipe = tokens >= b * (8 * tiles <= 19 * cus                      ? 400
                               : tiles > 3 * cus && 2 * tiles <= 7 * cus ? 1024
@@ -2323,12 +2326,9 @@ void launch_paged(const loom_paged_prefill_plan &p, const LongForm &form, dim3 g
     else
       hipLaunchKernelGGL((paged_prefill_pipe_kernel<4, 2, FP8>), grid, block, 0, stream, a);
   } else if (p.info.algorithm == LOOM_PAGED_PREFILL_LONG_TILE) {
-    if constexpr (!FP8)
-      if (p.tile_cols == 128) {
-        hipLaunchKernelGGL((paged_prefill_kernel<4, false, true, 2>), grid, block, 0, stream, a);
-        return;
-      }
-    if (form.groups == 2)
+    if (p.tile_cols == 128)
+      hipLaunchKernelGGL((paged_prefill_kernel<4, FP8, true, 2>), grid, block, 0, stream, a);
+    else if (form.groups == 2)
       hipLaunchKernelGGL((paged_prefill_kernel<8, FP8, true, 1>), grid, block, 0, stream, a);
     else
       hipLaunchKernelGGL((paged_prefill_kernel<4, FP8, true, 1>), grid, block, 0, stream, a);

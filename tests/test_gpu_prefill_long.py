@@ -311,3 +311,49 @@ def test_two_wave_groups_at_prompt_scale(L, oracle, n):
     res = paged_pair(L, 1, n, pool, hq, hkv, q, k, v, qo, ip, ix, last, tile="long")
     assert not np.any(np.isnan(oracle.bf16_to_f32(res[0][0])))
     log(f"  vs 16-column: {assert_close(oracle, res)}")
+
+
+# (kv-heads, requests, rows, tokens per request): commands on both sides of each
+# line between the pipelined and the plain tiles of 128 columns, grids of more
+# than two workgroups per CU
+FORMS = [
+    (8, 10, 130, 130),                            # short prompts, under a full round
+    (4, 5, 470, 470), (4, 4, 850, 850), (4, 6, 680, 680),  # longer ones: 2.3, 3.3, 4 per CU
+    (8, 4, 340, 700), (8, 5, 360, 720),           # contexts twice the rows: 2.7, 3.6
+    (8, 5, 215, 1500), (8, 6, 225, 1500), (8, 9, 215, 1500),  # long contexts: 2.2, 2.7, 3.9
+    (4, 2, 2100, 2100), (4, 2, 3300, 3300),       # two prompts: 4, 6.4
+]
+
+
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("form", FORMS, ids=lambda f: "x".join(map(str, f)))
+def test_forms_of_large_grids_match_row_tiles(L, oracle, form, fp8):
+    import torch
+    hkv, B, rows, n = form
+    hq = 8 * hkv
+    rng = np.random.default_rng(n)
+    kv_lens = [n - int(x) for x in rng.integers(0, 16, size=B)]
+    qo_lens = [min(rows, x) for x in kv_lens]
+    pages = [(x + 15) // 16 for x in kv_lens]
+    nnz, pool = sum(qo_lens), sum(pages) + 5
+    ip = np.concatenate([[0], np.cumsum(pages)]).astype(np.int32)
+    ix = rng.permutation(pool)[: ip[-1]].astype(np.int32)
+    last = np.array([x - (p - 1) * 16 for x, p in zip(kv_lens, pages)], np.int32)
+    qo = np.concatenate([[0], np.cumsum(qo_lens)]).astype(np.int32)
+    g = torch.Generator(device="cuda").manual_seed(nnz)
+    q = torch.randn(nnz * hq * 128, device="cuda", generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(pool * 16 * hkv * 128, device="cuda", generator=g).clamp(-3.75, 3.75)
+            for _ in range(2))
+    kw, scales = {}, None
+    if fp8:
+        kw, scales = {"kv_dtype": "fp8_e4m3"}, [0.8, 0.9]
+        k, v = (x.to(torch.float8_e4m3fn).view(torch.uint8) for x in (k, v))
+    else:
+        k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    p = L.PrefillProvider.load(0).plan_bf16_paged(
+        L.Bf16PagedPrefillSpec(B, nnz, pool, hq, hkv, **kw))
+    assert p.algorithm == "long_tile" and p.info.grid_blocks > 512
+    res = paged_pair(L, B, nnz, pool, hq, hkv, q, k, v, qo, ip, ix, last, spec_kw=kw,
+                     scales=scales, tile="long")
+    assert not np.any(np.isnan(oracle.bf16_to_f32(res[0][0])))
+    assert_close(oracle, res)
