@@ -268,3 +268,146 @@ def test_runs_of_tokens_that_score_minus_infinity(L, oracle, plan, form):
         r = ((at > 0.07) & (at < 0.21)) | ((at > 0.4) & (at < 0.45))
         return k.masked_fill(r, -3.0e38)
     assert_close(oracle, pipe_and_rows(L, oracle, plan, form, keys))
+
+
+def ragged_pair(L, hq, hkv, qo, kv, q, k, v):
+    """The long tiles' raw output bits and the 16-column algorithm's."""
+    import torch
+    from gpu_util import RaggedRunner, bf16_host, to_dev_i32
+    res = []
+    for tile in (0, 16):
+        r = RaggedRunner(L, len(qo) - 1, int(q.numel()) // (hq * 128), int(k.numel()) // (hkv * 128),
+                         hq, hkv, tile_cols=tile)
+        assert r.plan.algorithm == ("row_tile" if tile else "long_tile")
+        out, lse = r.run_dev(q, k, v, to_dev_i32(qo), to_dev_i32(kv))
+        res.append((bf16_host(out), lse.view(torch.int32).cpu().numpy()))
+    return res
+
+
+# (hq, hkv, qo_indptr, kv_indptr): ranges that overlap an earlier request's (the
+# later one owns the rest of its rows: tiles that do not begin at its first row),
+# one that ends before it begins, and requests with fewer keys than rows, whose
+# rows keep their sentinels; 64 and 128 columns
+GUARDED = [
+    (32, 8, [0, 400, 300, 700, 900], [0, 500, 600, 1300, 1400]),
+    (32, 8, [0, 900, 610, 1700, 2300], [0, 900, 1000, 2400, 2900]),
+    (28, 4, [0, 333, 1000, 777, 2100, 3000], [0, 433, 1100, 1200, 2800, 2900]),
+]
+
+
+@pytest.mark.parametrize("case", GUARDED, ids=lambda c: f"{c[0]}x{c[1]}_{c[2][-1]}")
+def test_ragged_rows_go_to_their_owners(L, oracle, case):
+    import torch
+    hq, hkv, qo, kv = case
+    g = torch.Generator(device="cuda").manual_seed(qo[-1])
+    q, k, v = (torch.randn(n * h * 128, device="cuda", generator=g).to(torch.bfloat16)
+               for n, h in ((qo[-1], hq), (kv[-1], hkv), (kv[-1], hkv)))
+    res = ragged_pair(L, hq, hkv, np.int32(qo), np.int32(kv), q, k, v)
+    dropped = np.isnan(oracle.bf16_to_f32(res[0][0])).reshape(qo[-1], -1)
+    rows = np.zeros(qo[-1], bool)
+    end = 0
+    for s0, s1, p0, p1 in zip(qo, qo[1:], kv, kv[1:]):
+        if s1 > max(s0, end) and not 0 < s1 - s0 <= p1 - p0:
+            rows[max(s0, end):s1] = True
+        end = max(end, s1)
+    assert rows.any() and np.array_equal(dropped.all(axis=1), rows)
+    assert_close(oracle, res)
+
+
+@pytest.mark.parametrize("hq,hkv,batch,most", [(64, 8, 70, 40), (64, 8, 130, 120)])
+def test_ragged_batches_past_a_wave(L, oracle, hq, hkv, batch, most):
+    """More than 64 requests: the workgroup-wide search, with a request past its
+    keys and one that overlaps the one before it."""
+    import torch
+    rng = np.random.default_rng(batch)
+    rows = rng.integers(most // 2 + 14, most + 14, size=batch)
+    kv = np.concatenate([[0], np.cumsum(rows + rng.integers(0, 9, size=batch))]).astype(np.int32)
+    qo = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    kv[67:] -= rows[66]              # request 66: fewer keys than rows
+    qo[33] += 7                      # request 32 takes the first rows of 33
+    kv[33:] += 7
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    q, k, v = (torch.randn(int(n) * h * 128, device="cuda", generator=g).to(torch.bfloat16)
+               for n, h in ((qo[-1], hq), (kv[-1], hkv), (kv[-1], hkv)))
+    res = ragged_pair(L, hq, hkv, qo, kv, q, k, v)
+    dropped = np.isnan(oracle.bf16_to_f32(res[0][0])).reshape(int(qo[-1]), -1).all(axis=1)
+    assert np.array_equal(np.nonzero(dropped)[0], np.arange(qo[66], qo[67]))
+    assert_close(oracle, res)
+
+
+def shifted(t, n):
+    """A copy of `t` that begins n elements into its allocation."""
+    import torch
+    x = torch.empty(t.numel() + n, dtype=t.dtype, device=t.device)
+    x[n:] = t
+    return x[n:]
+
+
+@pytest.mark.parametrize("form", ["bf16", "fp8", "ragged"])
+@pytest.mark.parametrize("rows", [600, 2500])
+def test_operands_on_four_byte_boundaries(L, oracle, rows, form):
+    """Q, K, V and O four bytes past a 16-byte boundary give the bits of the
+    aligned call: the tiles' loads straight into LDS and their row stores need no
+    more than four."""
+    import torch
+    from gpu_util import RaggedRunner, bf16_host, nan_bf16, to_dev_i32
+    hq, hkv, n = 32, 8, rows + 70
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    q, k, v = (torch.randn(m * h * 128, device="cuda", generator=g)
+               for m, h in ((rows, hq), (n + 26, hkv), (n + 26, hkv)))
+    q = q.to(torch.bfloat16)
+    by = 2
+    if form == "fp8":
+        k, v = (x[: (n + 26) // 16 * 16 * hkv * 128].to(torch.float8_e4m3fn).view(torch.uint8)
+                for x in (k, v))
+        by = 4
+    else:
+        k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    got = []
+    for move in (lambda x, m: x, shifted):
+        out = move(nan_bf16(rows * hq * 128), 2)
+        if form == "ragged":
+            r = RaggedRunner(L, 1, rows, n + 26, hq, hkv)
+            assert r.plan.algorithm == "long_tile"
+            o, l = r.run_dev(move(q, 2), move(k, by), move(v, by), to_dev_i32([0, rows]),
+                             to_dev_i32([0, n + 26]), out=out)
+        else:
+            pool = (n + 26) // 16
+            used = (n + 15) // 16
+            kk, vv = (x[: pool * 16 * hkv * 128] for x in (k, v))
+            r = PrefillRunner(L, 1, rows, pool, hq, hkv)
+            r.spec = L.Bf16PagedPrefillSpec(1, rows, pool, hq, hkv,
+                                            kv_dtype="fp8_e4m3" if form == "fp8" else "bf16")
+            r.plan = r.provider.plan_bf16_paged(r.spec)
+            assert r.plan.algorithm == "long_tile"
+            o, l = r.run_dev(move(q, 2), move(kk, by), move(vv, by), to_dev_i32([0, rows]),
+                             to_dev_i32([0, used]), to_dev_i32(np.arange(used)[::-1]),
+                             to_dev_i32([n - (used - 1) * 16]), out=out,
+                             scales=torch.tensor([0.8, 0.9], device="cuda") if form == "fp8" else None)
+        got.append((bf16_host(o.clone()), l.cpu().numpy()))
+    assert not np.any(np.isnan(oracle.bf16_to_f32(got[0][0])))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")], ids=["inf", "nan"])
+@pytest.mark.parametrize("plan,form", [(PLANS[0], "bf16"), (PLANS[3], "bf16"), (RAGGED[1], "ragged")],
+                         ids=["four_groups", "one_group", "ragged"])
+def test_infinite_and_nan_keys_stay_with_the_rows_that_see_them(L, oracle, plan, form, value):
+    """A key that is infinite or not a number in the last rows of each context
+    makes the rows that see it NaN, as in the 16-column algorithm, and leaves
+    every earlier row alone (a masked score is replaced whatever it was)."""
+    hq, hkv, qo_lens, kv_lens = plan[:4]
+
+    def keys(k, at):
+        n = np.repeat(kv_lens, kv_lens)
+        import torch
+        late = at[:, 0] * torch.from_numpy(n).to("cuda") > torch.from_numpy(n).to("cuda") - 20.5
+        return k.masked_fill(late[:, None], value)
+
+    res = pipe_and_rows(L, oracle, plan, form, keys)
+    bad = np.isnan(oracle.bf16_to_f32(res[0][0])).reshape(sum(qo_lens), -1)
+    want = np.concatenate([np.arange(r) >= r - 20 for r in qo_lens])
+    assert np.array_equal(bad.all(axis=1), want) and np.array_equal(bad.any(axis=1), want)
+    rows = np.repeat(~want, hq * 128)
+    (o, l), (eo, el) = res
+    assert_close(oracle, [(o[rows], l[np.repeat(~want, hq)]), (eo[rows], el[np.repeat(~want, hq)])])
