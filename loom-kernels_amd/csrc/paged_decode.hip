@@ -1857,9 +1857,9 @@ uint64_t loom_single_decode_split_k_workspace_bytes(const loom_single_decode_spl
 }
 
 namespace {
-// The split-K partial kernel and its merge.
-hipError_t launch_split_k(uint32_t group_tile, const DecodeArgs &a, int64_t L, int P, float *ws,
-                          hipStream_t stream) {
+// The split-K partial kernel, and its merge.
+hipError_t launch_split_k_partials(uint32_t group_tile, const DecodeArgs &a, int64_t L, int P,
+                                   float *ws, hipStream_t stream) {
   const uint64_t waves = (uint64_t)P * a.members;
   const dim3 g3((unsigned)((waves + kWaves - 1) / kWaves)), b3(kThreads);
   switch (group_tile) {
@@ -1868,10 +1868,11 @@ hipError_t launch_split_k(uint32_t group_tile, const DecodeArgs &a, int64_t L, i
     case 4: hipLaunchKernelGGL(single_decode_split_k_kernel<4>, g3, b3, 0, stream, a, L, P, ws); break;
     default: hipLaunchKernelGGL(single_decode_split_k_kernel<8>, g3, b3, 0, stream, a, L, P, ws); break;
   }
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  return hipGetLastError();
+}
+hipError_t launch_split_k_merge(const DecodeArgs &a, int P, const float *ws, hipStream_t stream) {
   hipLaunchKernelGGL(single_decode_split_k_merge_kernel, dim3((unsigned)a.hq), dim3(kMergeWaves * 64),
-                     0, stream, a, P, (const float *)ws);
+                     0, stream, a, P, ws);
   return hipGetLastError();
 }
 
@@ -1918,10 +1919,12 @@ loom_status_t loom_single_decode_enqueue(const loom_single_decode_plan_t *plan,
     // The partial states live in the queue's share states; where a command
     // may not use them the one-kernel form runs.
     const uint64_t bytes = s.num_query_heads * plan->partitions * loom::kStateWidth * 4;
-    if (uint8_t *ws = loom::queue_shares(scope, bytes))
-      return loom::record_launch(
-          scope, launch_split_k(plan->group_tile, a, L, (int)plan->partitions, (float *)ws, stream),
-          err);
+    if (float *ws = (float *)loom::queue_shares(scope, bytes)) {
+      const int P = (int)plan->partitions;
+      hipError_t e = launch_split_k_partials(plan->group_tile, a, L, P, ws, stream);
+      if (e == hipSuccess) e = launch_split_k_merge(a, P, ws, stream);
+      return loom::record_launch(scope, e, err);
+    }
   }
   const dim3 g3((unsigned)(s.num_kv_heads * plan->group_tiles)), b3(kThreads);
   switch (plan->group_tile) {
@@ -1966,21 +1969,11 @@ loom_status_t loom_single_decode_split_k_enqueue(const loom_single_decode_split_
                              l[5]->ptr);
   float *ws = (float *)l[3]->ptr;
   const int P = (int)plan->spec.partitions;
-  const uint64_t waves = (uint64_t)P * a.members;
-  const dim3 g3((unsigned)((waves + kWaves - 1) / kWaves)), b3(kThreads);
   hipStream_t stream = scope->queue->stream;
-  const int64_t L = (int64_t)s.kv_len;
-  switch (plan->group_tile) {
-    case 1: hipLaunchKernelGGL(single_decode_split_k_kernel<1>, g3, b3, 0, stream, a, L, P, ws); break;
-    case 2: hipLaunchKernelGGL(single_decode_split_k_kernel<2>, g3, b3, 0, stream, a, L, P, ws); break;
-    case 4: hipLaunchKernelGGL(single_decode_split_k_kernel<4>, g3, b3, 0, stream, a, L, P, ws); break;
-    default: hipLaunchKernelGGL(single_decode_split_k_kernel<8>, g3, b3, 0, stream, a, L, P, ws); break;
-  }
-  rc = loom::record_launch(scope, hipGetLastError(), err);
+  rc = loom::record_launch(
+      scope, launch_split_k_partials(plan->group_tile, a, (int64_t)s.kv_len, P, ws, stream), err);
   if (rc) return rc;
-  hipLaunchKernelGGL(single_decode_split_k_merge_kernel, dim3((unsigned)s.num_query_heads),
-                     dim3(kMergeWaves * 64), 0, stream, a, P, (const float *)ws);
-  return loom::record_launch(scope, hipGetLastError(), err);
+  return loom::record_launch(scope, launch_split_k_merge(a, P, ws, stream), err);
 }
 
 }  // extern "C"
