@@ -108,7 +108,7 @@ struct PrefillArgs {
 constexpr int kSplitState = 132;
 constexpr int kMaxSplits = 16;
 // Splits that a tile of `blocks` 16-row blocks uses of the command's `splits`:
-// at least eight blocks (two per wave) each.
+// one per eight blocks begun, so at least four blocks (one per wave) each.
 __host__ __device__ constexpr int tile_splits(int blocks, int splits) {
   const int most = (blocks + 7) / 8;
   return splits < most ? splits : most < 1 ? 1 : most;
@@ -894,7 +894,7 @@ struct LongWave {
   }
 };
 
-// ---- pipelined long tiles (LOOM_PAGED_PREFILL_LONG_TILE, 128 columns) -----------
+// ---- pipelined long tiles (LOOM_PAGED_PREFILL_LONG_TILE, 64 or 128 columns) -----
 // A workgroup owns 32 * NW flattened columns, two 16-column tiles per wave,
 // and walks the whole causal range in 32-token blocks (two 16-row blocks),
 // which are loaded straight into an LDS ring (buffer loads to LDS: no VGPRs or
@@ -910,10 +910,10 @@ struct LongWave {
 // next and the scores of the one after interleaved by hand (pin()); no maximum
 // per block; normalizer sums by dot products with ones; page addresses
 // computed per 64 blocks, one per lane; whole rows per load instruction.  Two
-// waves per SIMD (235 registers).  Tried with 32x32x16 MFMAs: a tenth faster
+// waves per SIMD (241-244 registers; FP8 pages 215-217).  Tried with 32x32x16 MFMAs: a tenth faster
 // on cool data (zeros), but their energy per flop is higher and random data
 // holds the card at its power limit from about 4096 rows on, where they lost 3%.
-// Measured against the plain long tiles: see the plan's rule.
+// Measured against the plain long tiles: see long_form.
 //
 // acc[t][e][i] = O[column of tile t][dim 16 e + 4 quad + i].
 //
@@ -1266,7 +1266,7 @@ constexpr int kLongTwoMinGrid = 512;
 template <int W, bool RAGGED, bool FP8, bool SH, int LT = 0, bool SPLIT = false>
 __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
   static_assert(!SPLIT || (!SH && !LT), "row tiles");
-  static_assert(!SH || W == 4 || (LT >= 1 && W == 8),
+  static_assert(!SH || W == 4 || (LT == 1 && W == 8),
                 "wide tiles: four waves; long tiles: four, or two groups of four with one tile");
   static_assert(!LT || SH, "long tiles: the wide tiles' columns");
   // Long tiles: four waves own the query tiles; G groups of them split the
@@ -1282,9 +1282,9 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
   }
   __shared__ PrefillSmem<W, SH, LT> sm;
   // long tiles: two K/V block slots per wave group (two groups: at least the
-  // merge staging of four waves' column states, 34 floats per lane and tile)
+  // merge staging of four waves' column states, 34 floats per lane)
   constexpr int kRingBytes = LT ? 2 * G * (FP8 ? 8192 : 16384) : 16;
-  constexpr int kMergeBytes = G == 2 ? LT * 34 * 4 * 64 * 4 : 0;
+  constexpr int kMergeBytes = G == 2 ? 34 * 4 * 64 * 4 : 0;
   __shared__ __align__(16) uint8_t lring[kRingBytes > kMergeBytes ? kRingBytes : kMergeBytes];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1518,37 +1518,29 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
       // Group 1 hands its column states to group 0 through the ring's LDS
       // (every wave is past its last ring read: block_or's barrier), and
       // group 0 merges them with its own, as the split-K merge does.
-      static_assert(LTT * 34 * 4 * 64 * 4 <= sizeof(lring), "merge staging fits the ring");
-      float *xs = reinterpret_cast<float *>(lring) + wq * (LTT * 34 * 64) + lane;
+      static_assert(34 * 4 * 64 * 4 <= sizeof(lring), "merge staging fits the ring");
+      float *x = reinterpret_cast<float *>(lring) + wq * (34 * 64) + lane;
       if (grp == 1) {
-#pragma unroll
-        for (int t = 0; t < LTT; ++t) {
-          float *x = xs + t * 34 * 64;
-          x[0] = lw.m_run[t];
-          x[64] = Lt[t];
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[(2 + 4 * e + i) * 64] = lw.acc[t][e][i];
-        }
-      }
-      __syncthreads();
-      if (grp == 1) return;
-#pragma unroll
-      for (int t = 0; t < LTT; ++t) {
-        const float *x = xs + t * 34 * 64;
-        const float m1 = x[0], l1 = x[64], m0 = lw.m_run[t];
-        const float M = fmaxf(m0, m1);
-        const float f0 = m0 == -INFINITY ? 0.0f : fast_exp2(m0 - M);
-        const float f1 = m1 == -INFINITY ? 0.0f : fast_exp2(m1 - M);
+        x[0] = lw.m_run[0];
+        x[64] = Lt[0];
 #pragma unroll
         for (int e = 0; e < 8; ++e)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            lw.acc[t][e][i] = lw.acc[t][e][i] * f0 + x[(2 + 4 * e + i) * 64] * f1;
-        Lt[t] = Lt[t] * f0 + l1 * f1;
-        lw.m_run[t] = M;
+          for (int i = 0; i < 4; ++i) x[(2 + 4 * e + i) * 64] = lw.acc[0][e][i];
       }
+      __syncthreads();
+      if (grp == 1) return;
+      const float m1 = x[0], l1 = x[64], m0 = lw.m_run[0];
+      const float M = fmaxf(m0, m1);
+      const float f0 = m0 == -INFINITY ? 0.0f : fast_exp2(m0 - M);
+      const float f1 = m1 == -INFINITY ? 0.0f : fast_exp2(m1 - M);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          lw.acc[0][e][i] = lw.acc[0][e][i] * f0 + x[(2 + 4 * e + i) * 64] * f1;
+      Lt[0] = Lt[0] * f0 + l1 * f1;
+      lw.m_run[0] = M;
     }
 #pragma unroll
     for (int t = 0; t < LTT; ++t) {
@@ -2011,7 +2003,7 @@ constexpr int kPrefillWavesPerEu = 3;
 // against two waves per SIMD (176 registers, no scratch): 975 against 869
 // TFLOP/s at 8192 rows, 822 against 695 at 4096.
 template <int W, bool FP8, bool SH = false, int LT = 0>
-__global__ __launch_bounds__(W * 64, LT ? (W == 8 ? (LT == 1 ? 4 : 2) : 3) : kPrefillWavesPerEu) void paged_prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(W * 64, LT ? (W == 8 ? 4 : 3) : kPrefillWavesPerEu) void paged_prefill_kernel(PrefillArgs a) {
   prefill_body<W, false, FP8, SH, LT>(a);
 }
 
@@ -2104,9 +2096,6 @@ loom_status_t prefill_grid(uint64_t batch, uint64_t nnz_qo, uint64_t hq, uint64_
 #ifndef LOOM_PREFILL_WIDE_MIN_GRID
 #define LOOM_PREFILL_WIDE_MIN_GRID 512
 #endif
-#ifndef LOOM_PREFILL_LONG_DEFAULT
-#define LOOM_PREFILL_LONG_DEFAULT 1
-#endif
 // The long tiles from a 64-column grid of this many workgroups: measured on
 // GQA4 32/8 prompts, 16.6 against 21.9 us (row tiles) at 1 x 512 rows (256
 // workgroups), 11.0 against 9.8 us at 1 x 256 (128).
@@ -2115,8 +2104,7 @@ loom_status_t prefill_grid(uint64_t batch, uint64_t nnz_qo, uint64_t hq, uint64_
 #endif
 loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
                                 uint64_t nnz_qo, uint64_t hq, uint64_t hkv, bool long_ok,
-                                bool long_default, uint32_t *tile_cols, bool *long_tile,
-                                loom_error_t *err) {
+                                uint32_t *tile_cols, bool *long_tile, loom_error_t *err) {
   const uint32_t t = flags & (LOOM_PLAN_PREFILL_TILE_16 | LOOM_PLAN_PREFILL_TILE_64 |
                               LOOM_PLAN_PREFILL_TILE_LONG);
   *long_tile = false;
@@ -2134,11 +2122,9 @@ loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
   const uint64_t cols = nnz_qo * (hq / hkv);
   const uint64_t grid64 = (cols / 64) * hkv;
   const bool long_requests = waves == 4 && batch > 0 && cols >= LOOM_PREFILL_WIDE_MIN_COLS * batch;
-  // Long prompts on BF16 pages take the long tiles, from a smaller grid than
-  // the wide tiles need (see the algorithm's measurements in the plan's
-  // documentation).
-  *long_tile = long_requests && long_default && LOOM_PREFILL_LONG_DEFAULT &&
-               grid64 >= LOOM_PREFILL_LONG_MIN_GRID;
+  // Long prompts take the long tiles, from a smaller grid than the wide tiles
+  // need.
+  *long_tile = long_requests && grid64 >= LOOM_PREFILL_LONG_MIN_GRID;
   if (*long_tile) {
     *tile_cols = (cols / 128) * hkv >= kLongTwoMinGrid ? 128 : 64;
     return LOOM_OK;
@@ -2154,20 +2140,23 @@ loom_status_t prefill_tile_cols(uint32_t flags, uint32_t waves, uint64_t batch,
 //    kv-head) wait for the CU's load path once more than one workgroup runs on
 //    a CU: whole rows (8 x 32 rows over 8192 tokens 159 | 112, over 512 14.9 |
 //    12.4; 2 x 100 over 2048 41.5 | 29.3; below, 3 x 13-24 over 220 7.1 | 7.7).
-//  - Long BF16 contexts of many requests, at memory speed (16 x 8 rows over
-//    8192 121 | 112, over 4096 51 | 45.5; FP8 pages 41 | 47: not taken;
-//    ragged within the runs' difference: not taken).
+//  - Long BF16 contexts of many requests, at memory speed: from 2/5 of the CUs in
+//    streams and 3/4 in tiles on (4-8 rows over 1024-8192: 16 requests 105 | 94,
+//    14 96 | 88, 13 88 | 87; 12, in streams below it, 77 | 85, and over 4200 42 |
+//    48); FP8 pages 41 | 47: not taken; ragged within the runs' difference: not
+//    taken.
 //  - Else the fragment order: with one workgroup per CU the stream is bound by
 //    what one CU keeps in flight (about 55 GB/s), and the turn through LDS
 //    adds 4-6 % (16 x 1 over 2048 23.4 | 25.9).
 //  - Few streams (requests x kv-heads) of long contexts leave most of the
 //    chip idle: shares of at least 32 blocks, up to two workgroups per CU
 //    (1 x 4 rows over 2048 22.7 | 14.9, over 8192 75 | 18, 8 x 4 FP8 over 8192
-//    76 | 39).  From 3/8 of the CUs on the unsplit streams already draw 5 TB/s
-//    (12 x 4 over 4096 41 | 50, 16 x 1 51 | 63), and a share pays for the merge
-//    (4-5 us).  Two shares of BF16 rows pay less: not for many requests whose
-//    tiles read K/V through different XCDs' L2 (kv-heads not a multiple of eight;
-//    16 x 6 rows over 4096 16/4 41 | 62, 4 x 42 over 4328 42 | 34).
+//    76 | 39; 12 x 4-8 over 1024-8192 77 | 60, all over 4200 42 | 44).  Past 3/8 of
+//    the CUs the unsplit streams already draw 5 TB/s (16 x 1 over 4096 51 | 63),
+//    and a share pays for the merge (4-5 us).  Two shares of BF16 rows pay less:
+//    not for many requests whose tiles read K/V through different XCDs' L2
+//    (kv-heads not a multiple of eight; 16 x 6 rows over 4096 16/4 41 | 62, 4 x 42
+//    over 4328 42 | 34).
 constexpr uint64_t kRowsLongBlocks = 256, kSplitMinBlocks = 128;
 template <bool RAGGED, bool FP8>
 int row_splits(uint64_t blocks, const PrefillArgs &a, uint64_t grid, int cus) {
@@ -2177,13 +2166,14 @@ int row_splits(uint64_t blocks, const PrefillArgs &a, uint64_t grid, int cus) {
   const uint64_t tiles =
       std::max<uint64_t>(batch, (uint64_t)a.nnz * a.group / 16 + batch / 2) * a.hkv;
   if (tiles >= 4 * streams && 2 * tiles >= 3 * chip) return 1;
-  if (!RAGGED && !FP8 && tiles >= chip && 2 * streams >= chip && avg >= kRowsLongBlocks) return 1;
-  if (avg < kSplitMinBlocks || 8 * streams >= 3 * chip ||
+  if (!RAGGED && !FP8 && 4 * tiles >= 3 * chip && 5 * streams >= 2 * chip && avg >= kRowsLongBlocks)
+    return 1;
+  if (avg < kSplitMinBlocks || 8 * streams > 3 * chip ||
       (4 * streams > chip && avg < kRowsLongBlocks))
     return 0;
   int s = kMaxSplits;
   while (s > 1 && ((uint64_t)s * 32 > avg || grid * s > 2 * chip)) s /= 2;
-  const bool two = avg >= kRowsLongBlocks && (FP8 || a.hkv % 8 == 0 || 8 * streams < chip);
+  const bool two = avg >= kRowsLongBlocks && (FP8 || a.hkv % 8 == 0 || 16 * streams < 3 * chip);
   return s >= 4 || (s == 2 && two) ? s : 0;
 }
 
@@ -2391,7 +2381,7 @@ loom_status_t loom_prefill_provider_plan_bf16_paged_options(
   uint32_t tile_cols = 16;
   bool long_tile = false;
   loom_status_t rc = prefill_tile_cols(opt.flags, waves, spec->batch_size, spec->nnz_qo,
-                                       spec->num_query_heads, spec->num_kv_heads, true, true,
+                                       spec->num_query_heads, spec->num_kv_heads, true,
                                        &tile_cols, &long_tile, err);
   if (rc) return rc;
   uint64_t tiles = 0, grid = 0;
@@ -2544,7 +2534,7 @@ loom_status_t loom_prefill_provider_plan_bf16_ragged(
   uint32_t tile_cols = 16;
   bool long_tile = false;
   loom_status_t rc = prefill_tile_cols(opt.flags, waves, spec->batch_size, spec->nnz_qo,
-                                       spec->num_query_heads, spec->num_kv_heads, false, true,
+                                       spec->num_query_heads, spec->num_kv_heads, false,
                                        &tile_cols, &long_tile, err);
   if (rc) return rc;
   uint64_t tiles = 0, grid = 0;
