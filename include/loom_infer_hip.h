@@ -719,9 +719,11 @@ typedef enum loom_paged_prefill_algorithm {
    * query fragments in registers and the softmax weights P rounded once to
    * BF16 for the P·V product (the normalizer is summed in FP32; within the
    * attention tolerance of the f32 reference; ragged: a BF16 high part and a
-   * residual).  64 or 128 columns per workgroup; plans whose grid leaves room
-   * for it run two or four groups of waves that split the K/V blocks and merge
-   * in LDS (block_threads 512).  No workspace. */
+   * residual).  64 or 128 columns per workgroup; commands whose grid leaves
+   * room for it run two or four groups of waves that split the K/V blocks and
+   * merge in LDS (block_threads 512).  An enqueue takes the faster of two
+   * kernels for the contexts that the bound page_indices hold; block_threads is
+   * that of contexts filling the pool.  No workspace. */
   LOOM_PAGED_PREFILL_LONG_TILE = 3
 } loom_paged_prefill_algorithm_t;
 

@@ -390,7 +390,7 @@ struct PrefillPage {
 
 // elem0: element offset of the block's first row for kv-head 0.  KROWS: K as
 // whole rows, in V's layout (staged through LDS before use): four rows per
-// load instruction take 18 cycles of the CU's load path, the fragment
+// load instruction take 21 cycles of the CU's load path, the fragment
 // layout's 16 rows 64.
 template <bool KROWS>
 __device__ __forceinline__ void load_prefill_page(PrefillPage &p, const PrefillArgs &a,
@@ -904,15 +904,17 @@ struct LongWave {
 // Bound and shape.  A 16x16x32 MFMA takes 16 cycles of the SIMD's matrix core
 // and holds its vector issue for 8 of them, an exponential for 8, other vector
 // instructions 4 (measured with register-only loops), and a wave issues in
-// order.  Per wave and block: 32 MFMAs (512 cycles), 16 exponentials and about
-// 35 other vector instructions, which fit beside the MFMAs only if they are
-// issued between them.  Hence: the products of one block, the softmax of the
+// order.  Per wave and block: 32 MFMAs (512 cycles) among 101 vector
+// instructions, 16 of them exponentials, which fit beside the MFMAs only if
+// they are issued between them (a block takes 1061 cycles of its SIMD at 8192
+// rows, so the matrix cores are busy 48%; the clock falls to 1.86 GHz).  Hence: the products of one block, the softmax of the
 // next and the scores of the one after interleaved by hand (pin()); no maximum
 // per block; normalizer sums by dot products with ones; page addresses
 // computed per 64 blocks, one per lane; whole rows per load instruction.  Two
-// waves per SIMD (241-244 registers; FP8 pages 215-217).  Tried with 32x32x16 MFMAs: a tenth faster
-// on cool data (zeros), but their energy per flop is higher and random data
-// holds the card at its power limit from about 4096 rows on, where they lost 3%.
+// waves per SIMD (241-244 registers; FP8 pages 215-217).  Tried with 32x32x16
+// MFMAs: a tenth faster on cool data (zeros), but their energy per flop is
+// higher and random data holds the card at its power limit from about 4096 rows
+// on, where they lost 3%.
 // Measured against the plain long tiles: see long_form.
 //
 // acc[t][e][i] = O[column of tile t][dim 16 e + 4 quad + i].
@@ -944,11 +946,12 @@ struct PipeWave {
   int kofs[4], vofs[4];  // the lane's fragments within a ring slot
 
   // Ring slot: 32 rows of K, then 32 of V, in 1 KB groups of whole rows (4;
-  // FP8 8), so that one load instruction covers whole rows (18 cycles of the
-  // CU's load path; 64 where each lane reads another row).  Within a group
+  // FP8 8), so that one load instruction covers whole rows (21 cycles of the
+  // CU's load path; 64 where it reads 64 bytes of each of 16).  Within a group
   // the 16-byte units of row r are permuted (BF16: unit u at u ^ 4 (r & 3);
-  // FP8: u ^ 2 ((r >> 1) & 3)) and the groups are padded, so that the fragment
-  // reads below fall on different banks.
+  // FP8: u ^ 2 ((r >> 1) & 3)) and the groups are padded, which spreads the
+  // fragment reads below over the banks (conflicts are 12% of the CU's cycles at
+  // 8192 rows).
   static constexpr int kRowBytes = FP8 ? 128 : 256;
   static constexpr int kUnits = kRowBytes / 16;
   static constexpr int kGroupRows = 1024 / kRowBytes;
@@ -1958,8 +1961,8 @@ __device__ __forceinline__ void pipe_body(const PrefillArgs &args) {
   // O through LDS (the ring is free; several groups: past a second barrier,
   // since other waves may still read the merge staging), each wave its own 32
   // rows of 256 bytes at a stride of kOutRow: whole rows then go out 16 bytes
-  // per lane (18 cycles of the CU's store path per KB; 8-byte pieces of 16 rows
-  // per instruction took 64, 2 us per workgroup of four waves).
+  // per lane (8-byte pieces of 16 rows per instruction took 2 us more per
+  // workgroup of four waves).
   if constexpr (G > 1) __syncthreads();
   static_assert(W * 32 * kOutRow <= sizeof(lring), "O staging");
   uint8_t *ot = lring + wave * 32 * kOutRow;
