@@ -255,3 +255,13 @@ def test_shared_commands_in_a_callers_capture(L, oracle):
             torch.cuda.synchronize()
             assert_close(oracle, [(bf16_host(o), l.view(torch.int32).cpu().numpy())
                                   for o, l in (held, outs)])
+
+
+def test_rows_at_the_most_shares(L, oracle):
+    """16 shares of each of 32 tiles fill the queue's buffer."""
+    case = (32, 8, [16], [8209], True)
+    kw, pool, scales, qkv, meta = case_inputs(case, "bf16")
+    here, scratch = paged(L, case, kw, pool, scales, qkv, meta)
+    there, _ = paged(L, case, kw, pool, scales, qkv, meta, waves=4)
+    assert scratch
+    assert_close(oracle, [here, there])

@@ -209,3 +209,13 @@ def test_tokens_that_score_minus_infinity(L, oracle, kv_len, partitions, first, 
                                v.reshape(kv_len, -1)[kept].ravel())
     out, lse = run_single(L, L.Bf16SingleDecodeSpec(kv_len, hq, hkv), q, k, v, partitions)
     compare_decode(oracle, out, lse, *ref)
+
+
+def test_direct_plan_at_its_most_partitions(L, oracle):
+    """131073 tokens of one kv-head: 1024 partitions of 8 heads, the most that the
+    queue's buffer holds for single decode."""
+    kv_len, hq, hkv = 131073, 8, 1
+    q, k, v = fixture(oracle, kv_len, hq, hkv, 0x7A11)
+    ref = oracle.single_decode(oracle.single_spec(kv_len, hq, hkv), q, k, v)
+    out, lse = run_single(L, L.Bf16SingleDecodeSpec(kv_len, hq, hkv), q, k, v)
+    compare_decode(oracle, out, lse, *ref)
