@@ -2227,6 +2227,10 @@ struct LongForm {
 // per CU (10 x 94-167 rows 64/8 20.6 / 22.3, 16 x 202-390 16/4 23.5 / 26.4).
 // Larger BF16 grids: two pipelined workgroups per CU or three plain ones.  The pipelined ones walk faster, but three rounds of them take what two
 // plain rounds take, and short contexts are all start and end:
+//  - Equal requests that fill their tiles, whose number is then known: pipe where
+//    its rounds are full, at two workgroups per CU (8 x 256 rows 17.6 / 16.5) and
+//    to four (8 x 512 40.2 / 38.0), plain to three (8 x 384 rows behind 1152
+//    75 / 87).
 //  - Whole prompts leave light tiles for the second round: pipe from 400 tokens
 //    on up to 19/8 workgroups per CU (4 x 348-642 rows 27.8 / 24.7), 650 to five
 //    (8 x 733-1216 16/4 63.1 / 56.5; 16 x 233-397 16/4 24.6 / 29.5), but 1024
@@ -2260,11 +2264,16 @@ LongForm long_form(const loom_paged_prefill_plan &p, uint64_t tokens) {
   const bool two_per_cu = grid <= 2 * cus, long_rows = nnz >= 1024 * b;
   const bool prefix = 2 * tokens >= 5 * nnz;
   const uint64_t page_rows = spec.page_size ? spec.page_size : loom::kPageSize;
+  bool even = false, one_round = two_per_cu;
   LongForm f{};
   if (p.tile_cols == 128) {
-    // workgroups that find a tile: every request's last tile is about half full
-    const uint64_t tiles = nnz * (spec.num_query_heads / hkv) / 128 * hkv + b * hkv / 2;
-    if (two_per_cu)
+    // workgroups that find a tile: every request's last tile is about half full,
+    // or whole where equal requests (chunks) fill it
+    const uint64_t cols = nnz * (spec.num_query_heads / hkv);
+    even = cols % (128 * b) == 0;
+    const uint64_t tiles = cols / 128 * hkv + (even ? 0 : b * hkv / 2);
+    one_round = tiles <= 2 * cus;
+    if (two_per_cu || (even && (one_round || (!fp8 && tiles > 3 * cus && tiles <= 4 * cus))))
       f.pipe = true;
     else if (fp8)
       f.pipe = 4 * tiles < 9 * cus || tiles > 3 * cus || tokens >= 420 * b;
@@ -2274,7 +2283,7 @@ LongForm long_form(const loom_paged_prefill_plan &p, uint64_t tokens) {
                                                                         : 650) &&
                (b == 1 || grid <= 5 * cus);
     else if (prefix)
-      f.pipe = 8 * tiles <= 19 * cus || (tiles > 3 * cus && tiles <= 5 * cus);
+      f.pipe = (!even && 8 * tiles <= 19 * cus) || (tiles > 3 * cus && tiles <= 5 * cus);
     else
       f.pipe = 4 * tiles > 13 * cus && 4 * tiles <= 17 * cus;
     f.groups = two_per_cu ? 2 : 1;
@@ -2298,9 +2307,11 @@ LongForm long_form(const loom_paged_prefill_plan &p, uint64_t tokens) {
   // +5%).  Two requests only on grids of more than six workgroups per CU (2 x
   // 4096 0 / -12%): below, unequal ones lose up to a quarter (1838 and 4101 rows
   // 28/4 155 -> 199).  Pipelined tiles behind long prefixes on BF16 pages, whose
-  // walks hardly differ, run request by request (11 x 193-381 rows behind
-  // 1816-5645 32/32 412 -> 310).
-  const bool by_request = f.pipe && !fp8 && !two_per_cu && p.tile_cols == 128 && prefix;
+  // walks hardly differ, run request by request from the second round on (11 x
+  // 193-381 rows behind 1816-5645 32/32 412 -> 310; in one round 4 x 512 behind
+  // 1536 62.6 -> 65.6).
+  const bool by_request =
+      f.pipe && !fp8 && p.tile_cols == 128 && prefix && !two_per_cu && !(even && one_round);
   f.interleave = b <= 16 && (b >= 3 || (b == 2 && grid > 6 * cus)) && !by_request;
   return f;
 }
