@@ -2225,8 +2225,9 @@ struct LongForm {
 // rows behind 2048-16384 tokens 473 / 384), and on FP8 pages, whose plain walk is
 // slower, unless requests of less than 420 tokens fill 9/4 to three workgroups
 // per CU (10 x 94-167 rows 64/8 20.6 / 22.3, 16 x 202-390 16/4 23.5 / 26.4).
-// Larger BF16 grids: two pipelined workgroups per CU or three plain ones.  The pipelined ones walk faster, but three rounds of them take what two
-// plain rounds take, and short contexts are all start and end:
+// Larger BF16 grids: two pipelined workgroups per CU or three plain ones.  The
+// pipelined ones walk faster, but three rounds of them take what two plain rounds
+// take, and short contexts are all start and end:
 //  - Equal requests that fill their tiles, whose number is then known: pipe where
 //    its rounds are full, at two workgroups per CU (8 x 256 rows 17.6 / 16.5) and
 //    to four (8 x 512 40.2 / 38.0), plain to three (8 x 384 rows behind 1152
